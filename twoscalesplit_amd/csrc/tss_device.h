@@ -226,6 +226,10 @@ enum { kTuneDensityLow = 0, kTuneDensityHigh, kTuneForceLow, kTuneForceHigh,
        kPairKernels };
 
 // Host-known launch parameters of one step.
+// Expected targets up to which a batch's neighbour sums take eight (four)
+// lanes per target.
+constexpr long long kCoop8Targets = 16384;
+constexpr long long kCoop4Targets = 49152;
 struct StepShape {
     int passes;               // radix passes
     int key_bits;
@@ -238,6 +242,7 @@ struct StepShape {
     int sort_grid;            // sort tiles launched (<= sort_tiles)
     int scan_tiles_l, scan_tiles_h, scan_tiles_g;  // compaction tiles launched
     PairTune tune[kPairKernels];
+    int coop;                 // neighbour sums: 8 or 4 lanes per target, 0: one (PairTune)
     int S;
     int red_slots;            // chunk slots in use (grid of the reduction)
     int list_parity;          // which list buffer holds the current lists

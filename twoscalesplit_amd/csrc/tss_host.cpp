@@ -227,6 +227,7 @@ struct tss_batch {
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     tss::PairTune tune[tss::kPairKernels] = {
         {256, 16, 0, 0}, {256, 16, 0, 0}, {256, 16, 0, 0}, {256, 16, 0, 0}};
+    bool shapes_set = false;        // launch shapes set by the caller
     long long cap_l = 0, cap_b = 0, ccl = 0, cch = 0;
     int max_scenes = 0;
     int sort_path = TSS_SORT_AUTO;  // grid-build sort (tss_set_grid_sort)
@@ -515,6 +516,21 @@ struct tss_batch {
             }
         if (resident != 1) sh.solo = -1;
         for (int k = 0; k < tss::kPairKernels; ++k) sh.tune[k] = tune[k];
+        // several lanes per target where one per target leaves the chip idle
+        // (and no launch shape was set by the caller), by the targets to
+        // expect: every low particle, twice as many under the reference
+        // rule. us per step with 1 / 4 / 8 lanes per target, one scene alone
+        // (and three at once, on their streams): plain 8k 114/84/77
+        // (41/31/29), 32k 115/89/90 (44/37/40), 48k 115/93/97 (46/44/46), 64k
+        // 118/104/110 (48/51/66); half split 8k 181/97/93 (65/38/39), 24k
+        // 189/120/131 (74/62/79), 32k 191/134/156 (75/74/97); all split 8k
+        // 167/98/100 (62/41/44), 24k 184/142/160 (73/72/93)
+        long long expect = 0;
+        for (const SceneHost& s : scenes)
+            if (s.alive) expect += (s.cfg.mode == TSS_MODE_REFERENCE ? 2LL : 1LL) * s.lcap;
+        sh.coop = shapes_set || expect > tss::kCoop4Targets ? 0
+                  : expect > tss::kCoop8Targets             ? 4
+                                                            : 8;
         sh.relax_iters = 0;
         for (auto& s : scenes)
             if (s.alive) sh.relax_iters = std::max(sh.relax_iters, s.cfg.relax_iters);
@@ -1012,6 +1028,7 @@ struct tss_batch {
     void set_tuning(const tss::PairTune* t) {
         for (int k = 0; k < tss::kPairKernels; ++k) validate_tune(t[k]);
         for (int k = 0; k < tss::kPairKernels; ++k) tune[k] = t[k];
+        shapes_set = true;
         update_shape();
     }
 
@@ -1029,6 +1046,9 @@ struct tss_batch {
         for (auto& x : scenes) alive += x.alive;
         require(alive > 0, "autotune: no scene");
         const bool was_timing = timing;
+        // the trials time one lane per target; a batch small enough for
+        // several goes back to those afterwards, which no shape beats there
+        const bool were_set = shapes_set;
         int dev = 0, cus = 0;
         HIP_CHECK(hipGetDevice(&dev));
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1114,6 +1134,8 @@ struct tss_batch {
                     best[k] = cand[c][k];
                 }
         set_tuning(best);
+        shapes_set = were_set;
+        update_shape();
         set_timing(was_timing);
         if (n_log) *n_log = logged;
         return taken;

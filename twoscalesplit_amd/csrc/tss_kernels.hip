@@ -1001,6 +1001,7 @@ __global__ void k_reorder(DevState d, const uint32_t* __restrict__ keys,
 }
 
 #include "tss_pairs.inc"
+#include "tss_coop.inc"
 
 // ---------------------------------------------------------------------------
 // Relaxation of the children injected by the last step's splits (the last
@@ -2502,13 +2503,19 @@ void launch_step(const DevState& d, const StepShape& sh, void* stream,
         k_relax_commit<<<gr, 256, 0, st>>>(d, d.list_h[par], it);
     }
     mark(1);
-    launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
-    mark(2);
-    launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh], 4 * sh.cap_alive, st);
-    mark(3);
-    launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
-    mark(4);
-    launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive, st);
+    if (sh.coop == 8)
+        launch_coop<8>(d, sh, vals, keys, st, ev == nullptr, mark);
+    else if (sh.coop == 4)
+        launch_coop<4>(d, sh, vals, keys, st, ev == nullptr, mark);
+    else {
+        launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
+        mark(2);
+        launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh], 4 * sh.cap_alive, st);
+        mark(3);
+        launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
+        mark(4);
+        launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive, st);
+    }
     mark(5);
     k_reduce<<<sh.red_slots, 256, 0, st>>>(d);
     mark(6);
