@@ -40,6 +40,8 @@ constexpr long long kSmallSortKeys = 65536;
 constexpr int kCellThreads = 256;
 constexpr int kCellTile = 1024;
 constexpr int kCountCellsPerKey = 4;
+// Cell tiles up to which a tile's base comes from the cells' counts
+constexpr int kCellDirect = 64;
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;  // entries per compaction tile
@@ -105,22 +107,21 @@ struct SceneCount {
     int cand;                 // split candidates of the last step
     int step;
     int seg_l0, seg_l1, seg_h0, seg_h1;  // sorted segments of the last step
-    // compaction prefixes at the scene's segment ends (kept low, kept high,
-    // admitted splits): counts = end - begin, no hot atomics
-    int kl0, kl1, kh0, kh1, sp0, sp1;
+    int drop_l, drop_h;       // listed entries that the last step removed
     int prom;                 // 1: a listed high particle is promoted (state 0)
     int act;                  // 1: a listed low particle is active (state 0)
     int hsurf;                // 1: a listed high particle is a free-surface particle
     unsigned long long psteps;  // particle-steps advanced since admission
 };
 
+// List sizes and flags, one per list parity: a step reads those of its parity
+// and its last launch writes the other.
 struct DevCounts {
     int n_l, n_h, n_g;        // lists the next step reads
-    int n_l_next, n_h_next, n_g_next;
     int n_l_last, n_h_last;   // lists the last step advanced (sorted sizes)
     // children injected by the last step's splits: the last n_fresh entries
     // of the high list (new children are appended after the kept ones)
-    int n_fresh, n_fresh_next;
+    int n_fresh;
     // 1: the step has a split candidate, promotion, merge or dissolve, or
     // the host changed the state since the last step; 0: every listed
     // entry is kept as it is (the compaction needs no flags). Reset to
@@ -141,7 +142,8 @@ struct DevState {
     int S;                    // scene capacity
     SceneDev* scenes;
     SceneCount* scnt;
-    DevCounts* counts;
+    DevCounts* counts;        // [2] by list parity (launchers: at_parity)
+    DevCounts* counts_next;
     int* scene_of;            // [CL] scene index of each low id (-1 free)
     float2* pos;
     float2* vel;
@@ -193,9 +195,8 @@ struct DevState {
     uint32_t* nmask;
     uint8_t* cand;            // [CL] split candidate flag per sorted low index
     uint8_t* merged;          // [CL] merged flag per low id
-    int* tile_sums;           // [2 * max_scan_tiles]
-    int* tile_base;           // [2 * max_scan_tiles]
-    int* seg_base;            // [8]
+    // [max_scan_tiles] per compaction tile: entries not kept, P1 entries
+    int2* tile_cnt;
     double* red;              // [red_slots * kRedFields]
     int* red_scene;           // [red_slots] scene of each chunk slot (-1 none)
     int* red_base;            // [S] first chunk slot of each scene
@@ -250,6 +251,9 @@ struct StepShape {
     int clear_blocks;         // blocks of the cell-table clear (clear_blk)
     int cap_binds;            // 1: a resident scene has cap_high < 4 cap_low
     int band_any;             // 1: a resident scene uses the surface band rule
+    int two;                  // 1: high particles or groups may be listed
+    int copy_only;            // 1: no entry can leave or join a list (not two,
+                              // and no raw device pointer handed out)
     int small_sort;           // 1: the resident capacity (5 cap_alive keys)
                               // fits kSmallSortKeys: one-workgroup sort
     int count_sort;           // 1: counting sort by cell (not small_sort,

@@ -228,6 +228,8 @@ struct tss_batch {
     tss::PairTune tune[tss::kPairKernels] = {
         {256, 16, 0, 0}, {256, 16, 0, 0}, {256, 16, 0, 0}, {256, 16, 0, 0}};
     bool shapes_set = false;        // launch shapes set by the caller
+    bool raw_ptr = false;           // a device pointer was handed out
+    bool high_seen = false;         // high particles or groups came from the host
     long long cap_l = 0, cap_b = 0, ccl = 0, cch = 0;
     int max_scenes = 0;
     int sort_path = TSS_SORT_AUTO;  // grid-build sort (tss_set_grid_sort)
@@ -308,7 +310,7 @@ struct tss_batch {
         d.S = max_scenes;
         d.scenes = dalloc<tss::SceneDev>(max_scenes, owned);
         d.scnt = dalloc<tss::SceneCount>(max_scenes, owned);
-        d.counts = dalloc<tss::DevCounts>(1, owned);
+        d.counts = dalloc<tss::DevCounts>(2, owned);
         d.scene_of = dalloc<int>(CL, owned);
         d.pos = dalloc<float2>(U, owned);
         d.vel = dalloc<float2>(U, owned);
@@ -352,9 +354,7 @@ struct tss_batch {
         d.merged = dalloc<uint8_t>(CL, owned);
         const int nst = (int)((CL + tss::kScanTile - 1) / tss::kScanTile) * 2 +
                         (int)((4 * CL + tss::kScanTile - 1) / tss::kScanTile);
-        d.tile_sums = dalloc<int>(2 * (size_t)nst, owned);
-        d.tile_base = dalloc<int>(2 * (size_t)nst, owned);
-        d.seg_base = dalloc<int>(8, owned);
+        d.tile_cnt = dalloc<int2>((size_t)nst, owned);
         red_cap = (int)((U + tss::kRedChunk - 1) / tss::kRedChunk) + max_scenes + 1;
         d.red = dalloc<double>((size_t)red_cap * tss::kRedFields, owned);
         d.red_scene = dalloc<int>(red_cap, owned);
@@ -371,7 +371,7 @@ struct tss_batch {
         // initial contents
         HIP_CHECK(hipMemsetAsync(d.scenes, 0, sizeof(tss::SceneDev) * max_scenes, stream));
         HIP_CHECK(hipMemsetAsync(d.scnt, 0, sizeof(tss::SceneCount) * max_scenes, stream));
-        HIP_CHECK(hipMemsetAsync(d.counts, 0, sizeof(tss::DevCounts), stream));
+        HIP_CHECK(hipMemsetAsync(d.counts, 0, 2 * sizeof(tss::DevCounts), stream));
         HIP_CHECK(hipMemsetAsync(d.cons, 0, sizeof(double) * 10 * max_scenes, stream));
         HIP_CHECK(hipMemsetAsync(d.red, 0, sizeof(double) * tss::kRedFields * red_cap, stream));
         HIP_CHECK(hipMemsetAsync(d.cflag, 0, 2 * (size_t)(ccl + cch), stream));
@@ -470,12 +470,19 @@ struct tss_batch {
             if (s.alive) cap += s.lcap;
         cap = std::max<long long>(cap, 1);
         const long long U = 5 * cap;
+        // high particles and groups: only where a two-scale scene makes them
+        // or the host listed some
+        sh.two = high_seen;
+        for (const SceneHost& s : scenes)
+            if (s.alive && s.cfg.mode != TSS_MODE_PLAIN) sh.two = 1;
+        sh.copy_only = !sh.two && !raw_ptr;
+        const long long live = sh.two ? U : cap;
         sh.cap_alive = cap;
-        sh.grid_elem = (int)std::min<long long>(kElemGridCap, (U + 255) / 256);
+        sh.grid_elem = (int)std::min<long long>(kElemGridCap, (live + 255) / 256);
         sh.sort_grid = (int)std::min<long long>(sh.sort_tiles, (U + tss::kSortTile - 1) / tss::kSortTile);
         sh.scan_tiles_l = (int)((cap + tss::kScanTile - 1) / tss::kScanTile);
-        sh.scan_tiles_h = (int)((4 * cap + tss::kScanTile - 1) / tss::kScanTile);
-        sh.scan_tiles_g = sh.scan_tiles_l;
+        sh.scan_tiles_h = sh.two ? (int)((4 * cap + tss::kScanTile - 1) / tss::kScanTile) : 0;
+        sh.scan_tiles_g = sh.two ? sh.scan_tiles_l : 0;
         sh.cap_binds = 0;
         sh.band_any = 0;
         for (const SceneHost& s : scenes) {
@@ -563,7 +570,7 @@ struct tss_batch {
 
     tss::DevCounts read_counts() {
         tss::DevCounts c;
-        HIP_CHECK(hipMemcpyAsync(&c, d.counts, sizeof(c), hipMemcpyDeviceToHost, stream));
+        HIP_CHECK(hipMemcpyAsync(&c, d.counts + sh.list_parity, sizeof(c), hipMemcpyDeviceToHost, stream));
         HIP_CHECK(hipStreamSynchronize(stream));
         return c;
     }
@@ -573,13 +580,13 @@ struct tss_batch {
     void write_counts(const tss::DevCounts& c) {
         tss::DevCounts w = c;
         w.events = 1;
-        HIP_CHECK(hipMemcpyAsync(d.counts, &w, sizeof(w), hipMemcpyHostToDevice, stream));
+        HIP_CHECK(hipMemcpyAsync(d.counts + sh.list_parity, &w, sizeof(w), hipMemcpyHostToDevice, stream));
         HIP_CHECK(hipStreamSynchronize(stream));
     }
 
     void mark_host_change() {
         const int one = 1;
-        HIP_CHECK(hipMemcpyAsync(&d.counts->events, &one, sizeof(int), hipMemcpyHostToDevice, stream));
+        HIP_CHECK(hipMemcpyAsync(&d.counts[sh.list_parity].events, &one, sizeof(int), hipMemcpyHostToDevice, stream));
         HIP_CHECK(hipStreamSynchronize(stream));
     }
 
@@ -1695,6 +1702,7 @@ struct tss_batch {
         // lists in unified ids; the scene's kept high entries go before the
         // batch's fresh tail and its own fresh entries after it, so every
         // scene's fresh children stay at the end of the high list
+        if (hd.n_high || hd.n_groups) set_high_seen();
         tss::DevCounts c = read_counts();
         const int par = sh.list_parity;
         const int CL = d.CL;
@@ -1742,6 +1750,12 @@ struct tss_batch {
         return sid;
     }
 
+    void set_high_seen() {
+        if (high_seen) return;
+        high_seen = true;
+        update_shape();
+    }
+
     void set_counts(int sid, int nl, int nh, int ng) {
         int alive = 0;
         for (auto& x : scenes) alive += x.alive;
@@ -1750,6 +1764,7 @@ struct tss_batch {
         require(nl >= 0 && nl <= s.lcap && nh >= 0 && nh <= 4 * s.lcap && ng >= 0 && ng <= s.lcap,
                 "counts out of range");
         tss::DevCounts c = read_counts();
+        if (nh || ng) set_high_seen();
         c.n_l = nl;
         c.n_h = nh;
         c.n_g = ng;
@@ -1886,8 +1901,13 @@ struct tss_batch {
         FieldView v = view(sid, field);
         require(v.kind == 0, "field has no plain device view");
         const int one[2] = {1, 1};
-        HIP_CHECK(hipMemcpyAsync(&d.counts->events, one, sizeof(one), hipMemcpyHostToDevice, stream));
+        HIP_CHECK(hipMemcpyAsync(&d.counts[sh.list_parity].events, one, sizeof(one),
+                                 hipMemcpyHostToDevice, stream));
         HIP_CHECK(hipStreamSynchronize(stream));
+        if (!raw_ptr) {
+            raw_ptr = true;
+            if (sh.copy_only) update_shape();
+        }
         return v.dev;
     }
 };

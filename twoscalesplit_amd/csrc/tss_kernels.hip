@@ -321,7 +321,8 @@ __global__ void k_fill_int(int* __restrict__ p, int v, long long n) {
 // cell (one atomic per run of equal keys along a wave's lanes) and the ids
 // are not copied (the scatter reads them from the lists). solo: the slot of
 // the only resident scene, or -1 (the scene then comes from scene_of).
-__global__ void k_begin_hash(DevState d, int nclear, int count, int solo,
+// ntiles: compaction tiles whose counters are cleared.
+__global__ void k_begin_hash(DevState d, int nclear, int count, int solo, int ntiles,
                              const int* __restrict__ list_l,
                              const int* __restrict__ list_h,
                              uint32_t* __restrict__ keys,
@@ -350,11 +351,14 @@ __global__ void k_begin_hash(DevState d, int nclear, int count, int solo,
             c.seg_l1 = 0;
             c.seg_h0 = 0;
             c.seg_h1 = 0;
-            c.kl0 = c.kl1 = c.kh0 = c.kh1 = c.sp0 = c.sp1 = 0;
+            c.drop_l = 0;
+            c.drop_h = 0;
             c.prom = 0;
             c.act = 0;
             c.hsurf = 0;
         }
+        for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < ntiles; t += nclear * blockDim.x)
+            d.tile_cnt[t] = make_int2(0, 0);
         return;
     }
     const int nl = d.counts->n_l;
@@ -404,13 +408,15 @@ __global__ void k_begin_hash(DevState d, int nclear, int count, int solo,
 // Counting sort by cell (replaces thrust::sort_by_key, R:2828-2834, with the
 // same stable order: by cell, ties by list position):
 //   k_begin_hash (count = 1) counts the keys per cell ->
-//   k_cell_sums (per tile of kCellTile cells) ->
+//   k_cell_sums (per tile of kCellTile cells; up to kCellDirect tiles
+//   k_cell_ranges reads the counts themselves) ->
 //   k_cell_ranges: each block sums the earlier tiles' sums (L2-resident,
 //   one read per tile) for its base; cstart = exclusive prefix of the
 //   counts (-1 for an empty cell), cend = cstart (the scatter's fill
 //   pointer), scene segments ->
 //   k_cell_scatter: list positions into their cell's range (atomic fill,
-//   any order within a cell; cend ends at cstart + count) ->
+//   any order within a cell; cend ends at cstart + count); resets the
+//   counts for the next grid build ->
 //   k_cell_reorder: each entry's rank among its cell's list positions gives
 //   its sorted position; then the cell-sorted copies.
 // The order within a cell is fixed by the rank, so the result is
@@ -438,12 +444,14 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_sums(DevState d, int ncel
 
 // Per tile: the counts to LDS (coalesced), each thread's kCellTile /
 // kCellThreads consecutive cells scanned in registers, the thread totals
-// scanned over the block, the prefixes written back through LDS. Resets the
-// counts for the next grid build. A scene's low and high cells are each one
+// scanned over the block, the prefixes written back through LDS. direct: the
+// tile's base from the earlier cells' counts (at most kCellDirect tiles: 16
+// KB per 4 tiles from L2, and a launch less), not from the tile sums. A
+// scene's low and high cells are each one
 // range of the unified cells (low ranges below CCL, high ranges above), so
 // a cell whose owner differs from its neighbour's, or that sits at either
 // side of CCL, bounds a range: it writes that scene's sorted segment bound.
-__global__ __launch_bounds__(kCellThreads) void k_cell_ranges(DevState d, int ncell) {
+__global__ __launch_bounds__(kCellThreads) void k_cell_ranges(DevState d, int ncell, int direct) {
     constexpr int kPer = kCellTile / kCellThreads;  // 4 cells per thread
     // one pad word per kPer: thread t's run starts at bank (t * 5) mod 32
     __shared__ int cells[kCellTile + kCellTile / kPer];
@@ -457,7 +465,17 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_ranges(DevState d, int nc
     // the tile's base: the sum of the earlier tiles' sums
     {
         int v = 0;
-        for (int q = t; q < (int)blockIdx.x; q += kCellThreads) v += d.ctile[q];
+        if (direct) {
+            // four cells per thread and tile, every load in flight
+            const int4* c4 = reinterpret_cast<const int4*>(d.ccount);
+#pragma unroll 8
+            for (int q = 0; q < (int)blockIdx.x; ++q) {
+                const int4 c = c4[q * (kCellTile / 4) + t];
+                v += (c.x + c.y) + (c.z + c.w);
+            }
+        } else {
+            for (int q = t; q < (int)blockIdx.x; q += kCellThreads) v += d.ctile[q];
+        }
         for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
         if ((t & 63) == 0) bsum[t >> 6] = v;
     }
@@ -507,7 +525,6 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_ranges(DevState d, int nc
         const int v = cnt[i] > 0 ? ex : -1;
         d.cstart[c] = v;
         d.cend[c] = v;
-        if (cnt[i] != 0) d.ccount[c] = 0;
         const int s = owner[x];
         if (s >= 0) {
             const bool high = c >= d.CCL;
@@ -535,11 +552,13 @@ __global__ __launch_bounds__(kCellThreads) void k_cell_ranges(DevState d, int nc
 __global__ void k_cell_scatter(DevState d, const uint32_t* __restrict__ keys,
                                const int* __restrict__ list_l,
                                const int* __restrict__ list_h,
-                               uint32_t* __restrict__ skeys) {
+                               uint32_t* __restrict__ skeys, int ncell) {
     const int nl = d.counts->n_l;
     const int n = nl + d.counts->n_h;
     const int stride = gridDim.x * blockDim.x;
     const int lane = threadIdx.x & 63;
+    // the cells' counts, read by k_cell_ranges, are zero for the next build
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncell; c += stride) d.ccount[c] = 0;
     for (int b0 = blockIdx.x * blockDim.x; b0 < n; b0 += stride) {
         const int k = b0 + (int)threadIdx.x;
         const bool valid = k < n;
@@ -1158,9 +1177,7 @@ __global__ void k_relax_commit(DevState d, const int* __restrict__ lh, int it) {
 // low, promoted high) and the max |v|^2 for the CFL time step. Fixed chunk
 // and tree shape -> bitwise reproducible, independent of other scenes.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_reduce(DevState d) {
-    __shared__ double sh[kRedFields][256];
-    const int slot = blockIdx.x;
+__device__ __forceinline__ void reduce_slot(const DevState& d, int slot, double (*sh)[256]) {
     const int s = d.red_scene[slot];
     if (s < 0) return;  // whole block: slot not owned by any scene
     const int chunk = slot - d.red_base[s];
@@ -1315,14 +1332,19 @@ __device__ bool in_band(const DevState& d, const SceneDev& sc, float2 x,
 }
 
 // Split candidates over the sorted low particles (R:1834-1836 rule or the
-// surface band rule).
-__global__ void k_split_cand(DevState d) {
+// surface band rule), with the entries that leave the low list because they
+// were deleted when the grid was built; both counted per scene and per
+// compaction tile (one atomic per wave where its lanes share a scene, the
+// usual case; a wave's 64 entries lie in one tile). block, nblocks: the
+// blocks of this part of the launch.
+__device__ __forceinline__ void split_candidates(const DevState& d, int block, int nblocks) {
     const int nl = d.counts->n_l;
-    GRID_STRIDE(k, nl) {
+    for (int k = block * (int)blockDim.x + (int)threadIdx.x; k < nl; k += nblocks * blockDim.x) {
         const int s = d.sscene[k];
         const SceneDev& sc = d.scenes[s];
+        const uint8_t st = d.sstate[k];
         uint8_t cand = 0;
-        if (sc.mode != 0 && d.sstate[k] == kActive) {
+        if (sc.mode != 0 && st == kActive) {
             if (sc.mode == 1) {
                 // predicted x' (R:1835): the force pass's post-step
                 // position, read in sorted order (the same value it
@@ -1333,20 +1355,33 @@ __global__ void k_split_cand(DevState d) {
             }
         }
         d.cand[k] = cand;
-        // per-scene candidate count; one atomic per wave when the wave's
-        // active lanes share a scene (the usual case)
+        const bool drop = st == kDeleted;
         const int s0 = __builtin_amdgcn_readfirstlane(s);
-        if (__ballot(s != s0) == 0ull) {
-            const uint64_t cm = __ballot(cand != 0);
-            const uint64_t act = __ballot(true);
-            const int lane = threadIdx.x & 63;
-            if (cm && lane == __ffsll((long long)act) - 1) {
-                atomicAdd(&d.scnt[s0].cand, (int)__popcll(cm));
-                d.counts->events = 1;
-            }
-        } else if (cand) {
-            atomicAdd(&d.scnt[s].cand, 1);
+        const uint64_t act = __ballot(true);
+        const bool first = (int)(threadIdx.x & 63) == __ffsll((long long)act) - 1;
+        const uint64_t cm = __ballot(cand != 0), dm = __ballot(drop);
+        if ((cm | dm) == 0ull) continue;
+        if (first) {
+            int2& t = d.tile_cnt[k / kScanTile];
+            if (dm) atomicAdd(&t.x, (int)__popcll(dm));
+            if (cm) atomicAdd(&t.y, (int)__popcll(cm));
             d.counts->events = 1;
+        }
+        if (__ballot(s != s0) == 0ull) {
+            if (first) {
+                SceneCount& c = d.scnt[s0];
+                if (dm) atomicAdd(&c.drop_l, (int)__popcll(dm));
+                if (cm) {
+                    atomicAdd(&c.cand, (int)__popcll(cm));
+                    atomicAdd(&c.n_split, (int)__popcll(cm));
+                }
+            }
+        } else {
+            if (drop) atomicAdd(&d.scnt[s].drop_l, 1);
+            if (cand) {
+                atomicAdd(&d.scnt[s].cand, 1);
+                atomicAdd(&d.scnt[s].n_split, 1);
+            }
         }
     }
 }
@@ -1380,11 +1415,18 @@ __device__ __forceinline__ float2 clamp_child(float2 ph, float2 pl, double rmax)
 // neighbourhoods of up to four children, one child per lane; the lanes of a
 // group sit in one wave and OR their results in a ballot, and lane 0
 // applies the decision. LANES = 1 tests the children in turn.
+// Entries that leave the lists here are counted per scene and compaction
+// tile (sidx is written where a band rule can remove any). th, tg: the first
+// compaction tile of the high and the group lists. thread, nthreads: of this
+// part of the launch.
 template <int LANES>
-__global__ void k_groups(DevState d, const int* __restrict__ list_g, int solo) {
+__device__ __forceinline__ void update_groups(const DevState& d, const uint32_t* __restrict__ vals,
+                                              const int* __restrict__ list_g, int solo, int th, int tg, int thread,
+                                              int nthreads) {
     static_assert(LANES == 1 || LANES == 4, "one lane or one per child");
+    const int nl = d.counts->n_l, nh = d.counts->n_h;
     const int ng = d.counts->n_g;
-    GRID_STRIDE(i, LANES * ng) {
+    for (int i = thread; i < LANES * ng; i += nthreads) {
         const int q = i / LANES, kl = i % LANES;
         const int p = list_g[q];
         // with one resident scene (solo >= 0), no lookup by id
@@ -1430,6 +1472,13 @@ __global__ void k_groups(DevState d, const int* __restrict__ list_g, int solo) {
                 for (int k = 0; k < 4; ++k) d.state[c0 + k] = 0;
                 atomicAdd(&d.scnt[s].n_promote, 1);
                 d.counts->events = 1;
+                // the parent leaves the low list (one that the list holds as
+                // deleted already is counted with the split candidates)
+                const uint32_t k = (uint32_t)d.sidx[p];
+                if (k < (uint32_t)nl && (int)vals[k] == p && d.sstate[k] != kDeleted) {
+                    atomicAdd(&d.tile_cnt[k / kScanTile].x, 1);
+                    atomicAdd(&d.scnt[s].drop_l, 1);
+                }
             } else if (sc.mode == 2 && !keep) {
                 // dissolve: children leave the lists, the parent stays
                 merged = 2;
@@ -1471,6 +1520,44 @@ __global__ void k_groups(DevState d, const int* __restrict__ list_g, int solo) {
             d.counts->events = 1;
         }
         d.merged[p] = merged;
+        if (merged) {
+            // the group and its listed children leave the lists
+            int2& t = d.tile_cnt[tg + q / kScanTile];
+            atomicAdd(&t.x, 1);
+            if (merged == 1) atomicAdd(&t.y, 1);
+            for (int c = 0; c < 4; ++c) {
+                const uint32_t k = (uint32_t)d.sidx[c0 + c] - (uint32_t)nl;
+                if (k < (uint32_t)nh && (int)vals[nl + k] == c0 + c) {
+                    atomicAdd(&d.tile_cnt[th + k / kScanTile].x, 1);
+                    atomicAdd(&d.scnt[s].drop_h, 1);
+                }
+            }
+        }
+    }
+}
+
+// What follows the force pass and does not depend on each other, in one
+// launch: blocks [0, nred) the reductions, the next nsplit the split
+// candidates, the others the groups. (Three launches took 8 + 4.5 + 4.5 us on
+// a small scene, one 8.)
+template <int LANES>
+__global__ __launch_bounds__(256) void k_adapt(DevState d, const uint32_t* __restrict__ vals,
+                                               const int* __restrict__ list_g, int solo, int nred,
+                                               int nsplit, int th, int tg) {
+    __shared__ double sh[kRedFields][256];
+    const int b = (int)blockIdx.x;
+    if (b < nred) {
+        reduce_slot(d, b, sh);
+    } else if (b < nred + nsplit) {
+        split_candidates(d, b - nred, nsplit);
+    } else {
+        // few groups and long band tests: a lane per child, and one wave per
+        // block to spread them over the CUs
+        constexpr int kUse = LANES == 4 ? 64 : 256;
+        if ((int)threadIdx.x < kUse)
+            update_groups<LANES>(d, vals, list_g, solo, th, tg,
+                                 (b - nred - nsplit) * kUse + (int)threadIdx.x,
+                                 ((int)gridDim.x - nred - nsplit) * kUse);
     }
 }
 
@@ -1481,11 +1568,12 @@ __global__ __launch_bounds__(256) void k_cap(DevState d) {
     __shared__ int part[256];
     const int s = blockIdx.x;
     const SceneDev& sc = d.scenes[s];
-    const SceneCount& c = d.scnt[s];
+    SceneCount& c = d.scnt[s];
     if (!sc.alive) return;
     const long long allowed_ll = ((long long)sc.cap_h - 4LL * c.n_g) / 4;
     const int allowed = allowed_ll < 0 ? 0 : (int)allowed_ll;
     if (c.cand <= allowed) return;
+    if (threadIdx.x == 0) c.n_split = allowed;
     int run = 0;
     for (int base = c.seg_l0; base < c.seg_l1; base += 256) {
         int k = base + threadIdx.x;
@@ -1499,7 +1587,10 @@ __global__ __launch_bounds__(256) void k_cap(DevState d) {
             __syncthreads();
         }
         int excl = run + part[threadIdx.x] - f;
-        if (f && excl >= allowed) d.cand[k] = 0;
+        if (f && excl >= allowed) {
+            d.cand[k] = 0;
+            atomicSub(&d.tile_cnt[k / kScanTile].y, 1);
+        }
         int tot = part[255];
         __syncthreads();
         run += tot;
@@ -1512,39 +1603,9 @@ __global__ __launch_bounds__(256) void k_cap(DevState d) {
 // [group tiles]; two counters per entry:
 //   P0 = keep (low: not deleted; high: group not merged; group: not merged)
 //   P1 = low: split admitted; group: merged.
+// k_adapt (and k_cap) left each tile's counts of entries not kept and of P1
+// in tile_cnt; a block sums those of the tiles before its own.
 // ---------------------------------------------------------------------------
-struct Flags {
-    int p0, p1;
-};
-
-__device__ __forceinline__ Flags entry_flags(const DevState& d,
-                                             const uint32_t* __restrict__ vals,
-                                             const int* __restrict__ list_g,
-                                             int seg, int i, int nl, int nh,
-                                             int ng) {
-    Flags f = {0, 0};
-    if (seg == 0) {
-        if (i < nl) {
-            int u = (int)vals[i];
-            f.p0 = d.state[u] != kDeleted;
-            f.p1 = d.cand[i];
-        }
-    } else if (seg == 1) {
-        if (i < nh) {
-            int u = (int)vals[nl + i];
-            f.p0 = !d.merged[(u - d.CL) >> 2];
-        }
-    } else {
-        if (i < ng) {
-            int p = list_g[i];
-            int m = d.merged[p];
-            f.p0 = m == 0;
-            f.p1 = m == 1;  // only merged-back parents are re-listed
-        }
-    }
-    return f;
-}
-
 __device__ __forceinline__ void tile_seg(const StepShape& sh, int tile,
                                          int& seg, int& t) {
     if (tile < sh.scan_tiles_l) {
@@ -1565,206 +1626,165 @@ __device__ __forceinline__ void tile_seg(const StepShape& sh, int tile,
 // ballots.
 constexpr int kScanWaves = kScanThreads / 64;
 
-__global__ __launch_bounds__(kScanThreads) void k_compact_reduce(
-    DevState d, StepShape sh, const uint32_t* __restrict__ vals,
-    const int* __restrict__ list_g) {
-    __shared__ int wsum[2][kScanWaves];
-    const int nl = d.counts->n_l, nh = d.counts->n_h, ng = d.counts->n_g;
-    int seg, t;
-    tile_seg(sh, blockIdx.x, seg, t);
-    // a tile past its segment's live entries counts nothing (the grid is
-    // sized by capacity): one write, and the whole block exits. A step
-    // without events keeps every live entry and splits or re-lists none:
-    // the counts follow from the segment sizes alone
-    const int nseg = seg == 0 ? nl : seg == 1 ? nh : ng;
-    if (t * kScanTile >= nseg || !d.counts->events) {
-        if (threadIdx.x == 0) {
-            d.tile_sums[2 * blockIdx.x] = max(0, min(kScanTile, nseg - t * kScanTile));
-            d.tile_sums[2 * blockIdx.x + 1] = 0;
-        }
-        return;
-    }
-    int a = 0, b = 0;  // wave totals (wave-uniform)
-    const int i0 = t * kScanTile + (int)threadIdx.x;
-    for (int q = 0; q < kScanItems; ++q) {
-        const Flags f = entry_flags(d, vals, list_g, seg, i0 + q * kScanThreads, nl, nh, ng);
-        a += __popcll(__ballot(f.p0));
-        b += __popcll(__ballot(f.p1));
-    }
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-        wsum[0][w] = a;
-        wsum[1][w] = b;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int ta = 0, tb = 0;
-        for (int v = 0; v < kScanWaves; ++v) {
-            ta += wsum[0][v];
-            tb += wsum[1][v];
-        }
-        d.tile_sums[2 * blockIdx.x] = ta;
-        d.tile_sums[2 * blockIdx.x + 1] = tb;
-    }
-}
+// P0 and P1 totals of the segments, and of the tiles of segment `seg` before
+// its tile `t`; the same on every thread. lds: 7 ints per wave.
+struct TileTotals {
+    int keep[3], p1[3];  // low, high, group
+    int before0, before1;
+};
 
-// Single block: exclusive scan of the tile sums, segment bases, new counts.
-// Only tiles holding live entries are scanned (the others count zero and
-// the scatter never reads their bases): virtual tile v runs over the live
-// tiles of the low, high and group segments in that order.
-__global__ __launch_bounds__(1024) void k_compact_top(DevState d, StepShape sh) {
-    __shared__ int2 part[1024];
-    __shared__ int2 seg_pre[2];  // prefixes where the high / group tiles start
-    const int th = sh.scan_tiles_l, tg = sh.scan_tiles_l + sh.scan_tiles_h;
+__device__ __forceinline__ TileTotals tile_totals(const DevState& d, const StepShape& sh, int seg,
+                                                  int t, int (*lds)[8]) {
     const DevCounts* c = d.counts;
-    const int ll = min((c->n_l + kScanTile - 1) / kScanTile, sh.scan_tiles_l);
-    const int lh = min((c->n_h + kScanTile - 1) / kScanTile, sh.scan_tiles_h);
-    const int lg = min((c->n_g + kScanTile - 1) / kScanTile, sh.scan_tiles_g);
-    const int nv = ll + lh + lg;
-    auto real = [&](int v) {
-        return v < ll ? v : (v < ll + lh ? th + (v - ll) : tg + (v - ll - lh));
-    };
-    const int per = (nv + 1023) / 1024;
-    const int t0 = threadIdx.x * per;
-    int a = 0, b = 0;
-    for (int i = 0; i < per; ++i) {
-        const int v = t0 + i;
-        if (v < nv) {
-            const int t = real(v);
-            a += d.tile_sums[2 * t];
-            b += d.tile_sums[2 * t + 1];
-        }
-    }
-    part[threadIdx.x] = make_int2(a, b);
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int2 w = threadIdx.x >= (unsigned)off ? part[threadIdx.x - off]
-                                              : make_int2(0, 0);
-        __syncthreads();
-        part[threadIdx.x].x += w.x;
-        part[threadIdx.x].y += w.y;
-        __syncthreads();
-    }
-    const int tot0 = part[1023].x, tot1 = part[1023].y;
-    if (threadIdx.x == 0) {
-        // a segment without live tiles starts at the total
-        seg_pre[0] = make_int2(tot0, tot1);
-        seg_pre[1] = make_int2(tot0, tot1);
-    }
-    __syncthreads();
-    int ra = part[threadIdx.x].x - a, rb = part[threadIdx.x].y - b;
-    for (int i = 0; i < per; ++i) {
-        const int v = t0 + i;
-        if (v < nv) {
-            const int t = real(v);
-            const int va = d.tile_sums[2 * t], vb = d.tile_sums[2 * t + 1];
-            if (v == ll) seg_pre[0] = make_int2(ra, rb);
-            if (v == ll + lh) seg_pre[1] = make_int2(ra, rb);
-            d.tile_base[2 * t] = ra;
-            d.tile_base[2 * t + 1] = rb;
-            ra += va;
-            rb += vb;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int b0h = seg_pre[0].x, b1h = seg_pre[0].y;
-        const int b0g = seg_pre[1].x, b1g = seg_pre[1].y;
-        const int keepL = b0h, nsplit = b1h;
-        const int keepH = b0g - b0h;
-        const int keepG = tot0 - b0g, nmerge = tot1 - b1g;
-        d.seg_base[0] = b0h;    // P0 base of high segment
-        d.seg_base[1] = b0g;    // P0 base of group segment
-        d.seg_base[2] = b1g;    // P1 base of group segment
-        d.seg_base[3] = keepL;
-        d.seg_base[4] = keepH;
-        d.seg_base[5] = keepG;
-        d.seg_base[6] = nsplit;
-        d.seg_base[7] = nmerge;
-        d.counts->n_l_next = keepL + nmerge;
-        d.counts->n_h_next = keepH + 4 * nsplit;
-        d.counts->n_fresh_next = 4 * nsplit;
-        d.counts->n_g_next = keepG + nsplit;
-    }
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_compact_scatter(
-    DevState d, StepShape sh, const uint32_t* __restrict__ vals,
-    const int* __restrict__ list_g, int* __restrict__ nlist_l,
-    int* __restrict__ nlist_h, int* __restrict__ nlist_g) {
-    __shared__ int wsum[2][kScanWaves];
-    const int nl = d.counts->n_l, nh = d.counts->n_h, ng = d.counts->n_g;
-    const bool events = d.counts->events != 0;
-    int seg, t;
-    tile_seg(sh, blockIdx.x, seg, t);
-    if (!events) {
-        // every live entry is kept, in order, and none splits or is
-        // re-listed: the next lists are copies of the sorted ids and the
-        // groups, and each scene's list bounds are its sorted segments
-        if (blockIdx.x == 0) {
-            for (int s = threadIdx.x; s < d.S; s += kScanThreads) {
-                SceneCount& c = d.scnt[s];
-                c.kl0 = c.seg_l0;
-                c.kl1 = c.seg_l1;
-                c.kh0 = c.seg_h0 - nl;
-                c.kh1 = c.seg_h1 - nl;
-                c.sp0 = 0;
-                c.sp1 = 0;
+    const int n[3] = {c->n_l, c->n_h, c->n_g};
+    const int first[3] = {0, sh.scan_tiles_l, sh.scan_tiles_l + sh.scan_tiles_h};
+    // entries not kept, P1 (high tiles have none), and both before tile t
+    int v[7] = {0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+        const int nt = (n[g] + kScanTile - 1) / kScanTile;
+        for (int q = (int)threadIdx.x; q < nt; q += kScanThreads) {
+            const int2 w = d.tile_cnt[first[g] + q];
+            v[g] += w.x;
+            if (g != 1) v[g == 0 ? 3 : 4] += w.y;
+            if (g == seg && q < t) {
+                v[5] += w.x;
+                v[6] += w.y;
             }
         }
-        const int nseg = seg == 0 ? nl : seg == 1 ? nh : ng;
-        const uint32_t* src = seg == 2 ? (const uint32_t*)list_g : vals + (seg == 1 ? nl : 0);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+#pragma unroll
+        for (int i = 0; i < 7; ++i) v[i] += __shfl_xor(v[i], off, 64);
+    }
+    const int w = (int)threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int i = 0; i < 7; ++i) lds[w][i] = v[i];
+    }
+    __syncthreads();
+    int tot[7];
+#pragma unroll
+    for (int i = 0; i < 7; ++i) {
+        tot[i] = 0;
+        for (int x = 0; x < kScanWaves; ++x) tot[i] += lds[x][i];
+    }
+    TileTotals r;
+    r.keep[0] = n[0] - tot[0];
+    r.keep[1] = n[1] - tot[1];
+    r.keep[2] = n[2] - tot[2];
+    r.p1[0] = tot[3];
+    r.p1[1] = 0;
+    r.p1[2] = tot[4];
+    r.before0 = t * kScanTile - tot[5];
+    r.before1 = tot[6];
+    return r;
+}
+
+// One tile of the next lists.
+__device__ __forceinline__ void compact_tile(const DevState& d, const StepShape& sh, int tile,
+                                             const uint32_t* __restrict__ vals,
+                                             const int* __restrict__ list_g,
+                                             int* __restrict__ nlist_l, int* __restrict__ nlist_h,
+                                             int* __restrict__ nlist_g, int (*lds)[8],
+                                             int (*wsum)[kScanItems][kScanWaves]) {
+    int seg, t;
+    tile_seg(sh, tile, seg, t);
+    const int n = seg == 0 ? d.counts->n_l : seg == 1 ? d.counts->n_h : d.counts->n_g;
+    // tiles past their segment's live entries (the grid is sized by
+    // capacity): whole block
+    if (t * kScanTile >= n) return;
+    const int i0 = t * kScanTile + (int)threadIdx.x;
+    const uint32_t* src = seg == 2 ? (const uint32_t*)list_g
+                                   : vals + (seg == 1 ? d.counts->n_l : 0);
+    // all of the thread's entries in flight
+    uint32_t u[kScanItems];
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q)
+        u[q] = src[min(i0 + q * kScanThreads, n - 1)];
+    if (sh.copy_only || !d.counts->events) {
+        // a step without events (no split, promotion, merge or dissolve, and
+        // no change from outside): every live entry is kept, in order, and
+        // none splits or is re-listed
         int* dst = seg == 0 ? nlist_l : seg == 1 ? nlist_h : nlist_g;
-        // all of the thread's entries in flight, then stored
-        uint32_t v[kScanItems];
 #pragma unroll
         for (int q = 0; q < kScanItems; ++q) {
-            const int i = t * kScanTile + q * kScanThreads + (int)threadIdx.x;
-            v[q] = i < nseg ? src[i] : 0u;
-        }
-#pragma unroll
-        for (int q = 0; q < kScanItems; ++q) {
-            const int i = t * kScanTile + q * kScanThreads + (int)threadIdx.x;
-            if (i < nseg) dst[i] = (int)v[q];
+            const int i = i0 + q * kScanThreads;
+            if (i < n) dst[i] = (int)u[q];
         }
         return;
     }
-    // tiles past their segment's live entries write nothing: whole block
-    if (t * kScanTile >= (seg == 0 ? nl : seg == 1 ? nh : ng)) return;
+    // the entries' flags, their loads in flight together: bit 0 P0, bit 1 P1
+    uint8_t f[kScanItems];
+    if (seg == 0) {
+        uint8_t st[kScanItems], s0[kScanItems], cd[kScanItems];
+#pragma unroll
+        for (int q = 0; q < kScanItems; ++q) {
+            const int i = min(i0 + q * kScanThreads, n - 1);
+            st[q] = d.state[u[q]];
+            s0[q] = d.sstate[i];
+            cd[q] = d.cand[i];
+        }
+#pragma unroll
+        for (int q = 0; q < kScanItems; ++q)
+            f[q] = (st[q] != kDeleted && s0[q] != kDeleted ? 1 : 0) | (cd[q] ? 2 : 0);
+    } else {
+        uint8_t m[kScanItems];
+#pragma unroll
+        for (int q = 0; q < kScanItems; ++q)
+            m[q] = d.merged[seg == 1 ? ((int)u[q] - d.CL) >> 2 : (int)u[q]];
+        // only merged-back parents are re-listed
+#pragma unroll
+        for (int q = 0; q < kScanItems; ++q)
+            f[q] = (m[q] == 0 ? 1 : 0) | (seg == 2 && m[q] == 1 ? 2 : 0);
+    }
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    uint64_t m0[kScanItems], m1[kScanItems];
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+        const bool live = i0 + q * kScanThreads < n;
+        m0[q] = __ballot(live && (f[q] & 1));
+        m1[q] = __ballot(live && (f[q] & 2));
+        if (lane == 0) {
+            wsum[0][q][wv] = __popcll(m0[q]);
+            wsum[1][q][wv] = __popcll(m1[q]);
+        }
+    }
+    const TileTotals tt = tile_totals(d, sh, seg, t, lds);  // a barrier inside
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    // output positions of the tile's first entry
-    int run0 = d.tile_base[2 * blockIdx.x];
-    int run1 = d.tile_base[2 * blockIdx.x + 1];
-    const int keepL = d.seg_base[3], keepH = d.seg_base[4],
-              keepG = d.seg_base[5];
-    // places entry i at output positions g0 / g1 (flags fq)
-    auto emit = [&](int i, int g0, int g1, const Flags& fq) {
-        if (seg == 0 && i < nl) {
-            const int u = (int)vals[i];
-            const int s = d.sscene[i];
-            SceneCount& sct = d.scnt[s];
-            // the scene's first / last sorted low entry
-            if (i == 0 || d.sscene[i - 1] != s) {
-                sct.kl0 = g0;
-                sct.sp0 = g1;
-            }
-            if (i == nl - 1 || d.sscene[i + 1] != s) {
-                sct.kl1 = g0 + fq.p0;
-                sct.sp1 = g1 + fq.p1;
-            }
-            if (fq.p0) nlist_l[g0] = u;
-            if (fq.p1) {
+    const int keepL = tt.keep[0], keepH = tt.keep[1], keepG = tt.keep[2];
+    int run0 = tt.before0, run1 = tt.before1;
+#pragma unroll
+    for (int q = 0; q < kScanItems; ++q) {
+        int pre0 = 0, pre1 = 0, tot0 = 0, tot1 = 0;
+        for (int v = 0; v < kScanWaves; ++v) {
+            const int c0 = wsum[0][q][v], c1 = wsum[1][q][v];
+            pre0 += v < wv ? c0 : 0;
+            pre1 += v < wv ? c1 : 0;
+            tot0 += c0;
+            tot1 += c1;
+        }
+        // exclusive output positions of this entry in its segment
+        const int g0 = run0 + pre0 + __popcll(m0[q] & lt);
+        const int g1 = run1 + pre1 + __popcll(m1[q] & lt);
+        run0 += tot0;
+        run1 += tot1;
+        const int i = i0 + q * kScanThreads;
+        if (i >= n) continue;
+        const int e = (int)u[q];
+        if (seg == 0) {
+            if (f[q] & 1) nlist_l[g0] = e;
+            if (f[q] & 2) {
                 // split (R:956-1005, 1834-1863): children at x' +-(rc, rc)
-                const SceneDev& sc = d.scenes[s];
-                nlist_g[keepG + g1] = u;
-                const float2 x = d.pos[u];
-                const float2 v = d.vel[u];
-                const float rho = d.rho[u];
+                const SceneDev& sc = d.scenes[d.sscene[i]];
+                nlist_g[keepG + g1] = e;
+                const float2 x = d.pos[e];
+                const float2 v = d.vel[e];
+                const float rho = d.rho[e];
                 const float two_rho = 2.0f * rho;
                 const float rc = (float)(0.5 * sqrt((double)sc.m_l /
                                                     ((double)two_rho * 3.14159265358979323846)));
-                const int c0 = d.CL + 4 * u;
+                const int c0 = d.CL + 4 * e;
                 for (int k = 0; k < 4; ++k) {
                     const int a2 = c0 + k;
                     d.pos[a2] = make_float2((k & 1) ? x.x - rc : x.x + rc,
@@ -1776,60 +1796,24 @@ __global__ __launch_bounds__(kScanThreads) void k_compact_scatter(
                     d.state[a2] = 1;
                     nlist_h[keepH + 4 * g1 + k] = a2;
                 }
-                d.state[u] = kTransient;
-                d.age[u] = 0;
+                d.state[e] = kTransient;
+                d.age[e] = 0;
             }
-        } else if (seg == 1 && i < nh) {
-            const int k = nl + i;
-            const int s = d.sscene[k];
-            SceneCount& sct = d.scnt[s];
-            const int gh = g0 - d.seg_base[0];
-            // the scene's first / last sorted high entry
-            if (k == nl || d.sscene[k - 1] != s) sct.kh0 = gh;
-            if (k == nl + nh - 1 || d.sscene[k + 1] != s) sct.kh1 = gh + fq.p0;
-            if (fq.p0) nlist_h[gh] = (int)vals[k];
-        } else if (seg == 2 && i < ng) {
-            const int p = list_g[i];
-            if (fq.p0) nlist_g[g0 - d.seg_base[1]] = p;
-            if (fq.p1) nlist_l[keepL + (g1 - d.seg_base[2])] = p;
+        } else if (seg == 1) {
+            if (f[q] & 1) nlist_h[g0] = e;
+        } else {
+            if (f[q] & 1) nlist_g[g0] = e;
+            if (f[q] & 2) nlist_l[keepL + g1] = e;
         }
-    };
-    for (int q = 0; q < kScanItems; ++q) {
-        const int i = t * kScanTile + q * kScanThreads + (int)threadIdx.x;
-        const Flags fq = entry_flags(d, vals, list_g, seg, i, nl, nh, ng);
-        const uint64_t m0 = __ballot(fq.p0), m1 = __ballot(fq.p1);
-        if (lane == 0) {
-            wsum[0][wv] = __popcll(m0);
-            wsum[1][wv] = __popcll(m1);
-        }
-        __syncthreads();
-        int pre0 = 0, pre1 = 0, tot0 = 0, tot1 = 0;
-        for (int v = 0; v < kScanWaves; ++v) {
-            const int c0 = wsum[0][v], c1 = wsum[1][v];
-            pre0 += v < wv ? c0 : 0;
-            pre1 += v < wv ? c1 : 0;
-            tot0 += c0;
-            tot1 += c1;
-        }
-        __syncthreads();  // wsum is rewritten by the next chunk
-        // exclusive output positions of this entry
-        const int g0 = run0 + pre0 + __popcll(m0 & lt);
-        const int g1 = run1 + pre1 + __popcll(m1 & lt);
-        run0 += tot0;
-        run1 += tot1;
-        emit(i, g0, g1, fq);
     }
 }
 
-// ---------------------------------------------------------------------------
-// End of step: per-scene dt, conservation sums and counters; global counts.
-// ---------------------------------------------------------------------------
-// One block per scene: the scene's chunk partials are summed in a fixed
-// order (thread t takes slots t, t+256, ...; then a fixed tree), so the
+// End of step of one scene: dt, conservation sums and counters; with scene 0
+// the next step's list sizes. The scene's chunk partials are summed in a
+// fixed order (thread t takes slots t, t+256, ...; then a fixed tree), so the
 // sums are bitwise reproducible.
-__global__ __launch_bounds__(256) void k_finalize(DevState d) {
-    __shared__ double sh[kRedFields][256];
-    const int s = blockIdx.x;
+__device__ __forceinline__ void finalize_scene(const DevState& d, const StepShape& shp, int s,
+                                               double (*sh)[256], int (*lds)[8]) {
     SceneDev& sc = d.scenes[s];
     SceneCount& c = d.scnt[s];
     const int nslots = d.red_n[s];
@@ -1881,13 +1865,12 @@ __global__ __launch_bounds__(256) void k_finalize(DevState d) {
         c.n_h_last = c.seg_h1 - c.seg_h0;
         c.psteps += (unsigned long long)(c.n_l_last + c.n_h_last);
         // next lists: low = kept + merged; high = kept + 4 per split
-        c.n_split = c.sp1 - c.sp0;
-        c.n_l = (c.kl1 - c.kl0) + c.n_merge;
-        c.n_h = (c.kh1 - c.kh0) + 4 * c.n_split;
+        c.n_l = c.n_l_last - c.drop_l + c.n_merge;
+        c.n_h = c.n_h_last - c.drop_h + 4 * c.n_split;
         c.n_g = c.n_g + c.n_split - c.n_merge - c.n_dissolve;
         c.step += 1;
         // rounding bound of the sums: per-term rounding (<= 2u) + the
-        // serial per-thread loop + 8-level tree of k_reduce, then the
+        // serial per-thread loop + 8-level tree of the chunk sums, then the
         // per-thread slot loop + 8-level tree here
         const double serial = (double)(kRedChunk / 256);
         const double kk = serial + 8.0 + (double)((nslots + 255) / 256) + 8.0 + 2.0;
@@ -1907,16 +1890,43 @@ __global__ __launch_bounds__(256) void k_finalize(DevState d) {
             sc.dt = (float)dt;
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        DevCounts& g = *d.counts;
-        g.n_l_last = g.n_l;
-        g.n_h_last = g.n_h;
-        g.n_l = g.n_l_next;
-        g.n_h = g.n_h_next;
-        g.n_g = g.n_g_next;
-        g.n_fresh = g.n_fresh_next;
-        g.events = g.events_floor;
+    if (s == 0) {
+        const bool events = !shp.copy_only && d.counts->events != 0;
+        TileTotals t{};
+        if (events) t = tile_totals(d, shp, 0, 0, lds);
+        if (threadIdx.x == 0) {
+            DevCounts g = *d.counts;
+            g.n_l_last = g.n_l;
+            g.n_h_last = g.n_h;
+            g.n_fresh = 0;
+            if (events) {
+                g.n_l = t.keep[0] + t.p1[2];
+                g.n_h = t.keep[1] + 4 * t.p1[0];
+                g.n_g = t.keep[2] + t.p1[0];
+                g.n_fresh = 4 * t.p1[0];
+            }
+            g.events = g.events_floor;
+            *d.counts_next = g;
+        }
     }
+}
+
+// The next lists and the end of the step in one launch: blocks [0, nfin) end
+// the step of a scene each, the others write a compaction tile each. Neither
+// reads what the other writes (the counts are those of the other list
+// parity).
+__global__ __launch_bounds__(kScanThreads) void k_end_step(
+    DevState d, StepShape sh, int nfin, const uint32_t* __restrict__ vals,
+    const int* __restrict__ list_g, int* __restrict__ nlist_l, int* __restrict__ nlist_h,
+    int* __restrict__ nlist_g) {
+    __shared__ double red[kRedFields][256];
+    __shared__ int lds[kScanWaves][8];
+    __shared__ int wsum[2][kScanItems][kScanWaves];
+    if ((int)blockIdx.x < nfin)
+        finalize_scene(d, sh, (int)blockIdx.x, red, lds);
+    else
+        compact_tile(d, sh, (int)blockIdx.x - nfin, vals, list_g, nlist_l, nlist_h, nlist_g, lds,
+                     wsum);
 }
 
 // ---------------------------------------------------------------------------
@@ -2115,19 +2125,20 @@ __global__ __launch_bounds__(kScanThreads) void k_filter_count(
             ta += wsum[0][v];
             tf += wsum[1][v];
         }
-        d.tile_sums[2 * blockIdx.x] = ta;
-        d.tile_sums[2 * blockIdx.x + 1] = tf;
+        d.tile_cnt[blockIdx.x] = make_int2(ta, tf);
     }
 }
 
 // One block: per segment, exclusive prefix of the tiles' kept counts (the
-// tiles' output bases) and the segment's new size; the high segment's kept
-// fresh entries give the new n_fresh.
+// tiles' output bases, in their place) and the segment's new size; the high
+// segment's kept fresh entries give the new n_fresh. The new counts are those
+// of the other list parity.
 __global__ __launch_bounds__(1024) void k_filter_top(DevState d, StepShape sh) {
     __shared__ int part[1024];
     const int start[3] = {0, sh.scan_tiles_l, sh.scan_tiles_l + sh.scan_tiles_h};
     const int len[3] = {sh.scan_tiles_l, sh.scan_tiles_h, sh.scan_tiles_g};
     int fresh = 0;
+    DevCounts next = *d.counts;
     for (int sg = 0; sg < 3; ++sg) {
         const int nt = len[sg];
         const int per = (nt + 1023) / 1024;
@@ -2135,8 +2146,8 @@ __global__ __launch_bounds__(1024) void k_filter_top(DevState d, StepShape sh) {
         int a = 0, f = 0;
         for (int i = 0; i < per; ++i) {
             if (t0 + i < nt) {
-                a += d.tile_sums[2 * (start[sg] + t0 + i)];
-                f += d.tile_sums[2 * (start[sg] + t0 + i) + 1];
+                a += d.tile_cnt[start[sg] + t0 + i].x;
+                f += d.tile_cnt[start[sg] + t0 + i].y;
             }
         }
         part[threadIdx.x] = a;
@@ -2151,9 +2162,9 @@ __global__ __launch_bounds__(1024) void k_filter_top(DevState d, StepShape sh) {
         const int tot = part[1023];
         for (int i = 0; i < per; ++i) {
             if (t0 + i < nt) {
-                const int tt = start[sg] + t0 + i;
-                const int v = d.tile_sums[2 * tt];
-                d.tile_base[2 * tt] = run;
+                int2& w = d.tile_cnt[start[sg] + t0 + i];
+                const int v = w.x;
+                w.x = run;
                 run += v;
             }
         }
@@ -2168,17 +2179,15 @@ __global__ __launch_bounds__(1024) void k_filter_top(DevState d, StepShape sh) {
             }
             fresh = part[0];
         }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            if (sg == 0) d.counts->n_l = tot;
-            if (sg == 1) {
-                d.counts->n_h = tot;
-                d.counts->n_fresh = fresh;
-            }
-            if (sg == 2) d.counts->n_g = tot;
+        if (sg == 0) next.n_l = tot;
+        if (sg == 1) {
+            next.n_h = tot;
+            next.n_fresh = fresh;
         }
+        if (sg == 2) next.n_g = tot;
         __syncthreads();
     }
+    if (threadIdx.x == 0) *d.counts_next = next;
 }
 
 __global__ __launch_bounds__(kScanThreads) void k_filter_scatter(
@@ -2188,15 +2197,13 @@ __global__ __launch_bounds__(kScanThreads) void k_filter_scatter(
     __shared__ int wsum[kScanWaves];
     int seg, t;
     tile_seg(sh, blockIdx.x, seg, t);
-    // the segment sizes before the filter (k_filter_top has rewritten the
-    // counts): passed by the host, which read them before the launch
     const int n = seg == 0 ? n_l : seg == 1 ? n_h : n_g;
     if (t * kScanTile >= n) return;  // whole block
     const int* L = seg == 0 ? ll : seg == 1 ? lh : lg;
     int* O = seg == 0 ? nll : seg == 1 ? nlh : nlg;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    int run = d.tile_base[2 * blockIdx.x];
+    int run = d.tile_cnt[blockIdx.x].x;
     for (int q = 0; q < kScanItems; ++q) {
         const int i = t * kScanTile + q * kScanThreads + (int)threadIdx.x;
         const int v = i < n ? L[i] : 0;
@@ -2440,6 +2447,14 @@ void launch_fill_int(int* p, int value, long long n, void* stream) {
     k_fill_int<<<blocks_for(n, 256, 4096), 256, 0, st>>>(p, value, n);
 }
 
+// The state with the counts of a list parity (and of the other one).
+static DevState at_parity(const DevState& d, int par) {
+    DevState e = d;
+    e.counts = d.counts + par;
+    e.counts_next = d.counts + (par ^ 1);
+    return e;
+}
+
 // Grid build: clears, hash, sort, ranges + reorder. Returns the buffer index
 // holding the sorted keys/vals.
 // with_sidx: also the sorted index of each id (sidx), which only the band
@@ -2449,13 +2464,15 @@ static int enqueue_grid(const DevState& d, const StepShape& sh,
                         hipStream_t st, int with_sidx) {
     const int par = sh.list_parity;
     k_begin_hash<<<sh.clear_blocks + sh.grid_elem, 256, 0, st>>>(
-        d, sh.clear_blocks, sh.count_sort, sh.solo, d.list_l[par], d.list_h[par], d.keys[0],
-        d.vals[0]);
+        d, sh.clear_blocks, sh.count_sort, sh.solo,
+        sh.scan_tiles_l + sh.scan_tiles_h + sh.scan_tiles_g, d.list_l[par], d.list_h[par],
+        d.keys[0], d.vals[0]);
     if (sh.count_sort) {
-        k_cell_sums<<<sh.cell_tiles, kCellThreads, 0, st>>>(d, sh.key_cells);
-        k_cell_ranges<<<sh.cell_tiles, kCellThreads, 0, st>>>(d, sh.key_cells);
+        const int direct = sh.cell_tiles <= kCellDirect;
+        if (!direct) k_cell_sums<<<sh.cell_tiles, kCellThreads, 0, st>>>(d, sh.key_cells);
+        k_cell_ranges<<<sh.cell_tiles, kCellThreads, 0, st>>>(d, sh.key_cells, direct);
         k_cell_scatter<<<sh.grid_elem, 256, 0, st>>>(d, d.keys[0], d.list_l[par],
-                                                     d.list_h[par], d.keys[1]);
+                                                     d.list_h[par], d.keys[1], sh.key_cells);
         k_cell_reorder<<<sh.grid_elem, 256, 0, st>>>(d, d.keys[1], d.vals[1], with_sidx);
         return 1;
     }
@@ -2480,12 +2497,13 @@ static int enqueue_grid(const DevState& d, const StepShape& sh,
 }
 
 void launch_grid_only(const DevState& d, const StepShape& sh, void* stream) {
-    enqueue_grid(d, sh, (hipStream_t)stream, 0);
+    enqueue_grid(at_parity(d, sh.list_parity), sh, (hipStream_t)stream, 0);
 }
 
-void launch_step(const DevState& d, const StepShape& sh, void* stream,
+void launch_step(const DevState& base, const StepShape& sh, void* stream,
                  void* timing_events, unsigned int event_flags) {
     hipStream_t st = (hipStream_t)stream;
+    const DevState d = at_parity(base, sh.list_parity);
     hipEvent_t* ev = (hipEvent_t*)timing_events;
     // event points: see kTimingPoints (tss_device.h)
     auto mark = [&](int k) {
@@ -2510,36 +2528,55 @@ void launch_step(const DevState& d, const StepShape& sh, void* stream,
     else {
         launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
         mark(2);
-        launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh], 4 * sh.cap_alive, st);
+        if (sh.two)
+            launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh], 4 * sh.cap_alive,
+                                     st);
         mark(3);
         launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
         mark(4);
-        launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive, st);
+        if (sh.two)
+            launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive, st);
     }
     mark(5);
-    k_reduce<<<sh.red_slots, 256, 0, st>>>(d);
-    mark(6);
-    k_split_cand<<<sh.grid_elem, 256, 0, st>>>(d);
-    // few groups and long band tests: a lane per child, small blocks to
-    // spread them over the CUs
-    if (sh.band_any)
-        k_groups<4><<<blocks_for(4 * sh.cap_alive, 64, 16384), 64, 0, st>>>(d, d.list_g[par],
-                                                                           sh.solo);
-    else
-        k_groups<1><<<blocks_for(sh.cap_alive, 256, 4096), 256, 0, st>>>(d, d.list_g[par],
-                                                                         sh.solo);
+    // the reductions, split candidates and groups in one launch (two where
+    // the phases are timed); nothing splits without a two-scale scene
+    const int nsplit = sh.copy_only ? 0 : blocks_for(sh.cap_alive, 256, 32768);
+    const int ngroup = !sh.two ? 0
+                       : sh.band_any ? blocks_for(4 * sh.cap_alive, 64, 16384)
+                                     : blocks_for(sh.cap_alive, 256, 4096);
+    const int th = sh.scan_tiles_l, tg = sh.scan_tiles_l + sh.scan_tiles_h;
+    auto adapt = [&](int nred, int ns, int ng) {
+        if (nred + ns + ng == 0) return;
+        if (sh.band_any)
+            k_adapt<4><<<nred + ns + ng, 256, 0, st>>>(d, vals, d.list_g[par], sh.solo, nred, ns,
+                                                       th, tg);
+        else
+            k_adapt<1><<<nred + ns + ng, 256, 0, st>>>(d, vals, d.list_g[par], sh.solo, nred, ns,
+                                                       th, tg);
+    };
+    if (ev) {
+        adapt(sh.red_slots, 0, 0);
+        mark(6);
+        adapt(0, nsplit, ngroup);
+    } else {
+        adapt(sh.red_slots, nsplit, ngroup);
+    }
     // the cap can bind only where cap_high < 4 cap_low: a scene's groups
     // and candidates never exceed its low ids
     if (sh.cap_binds) k_cap<<<sh.S, 256, 0, st>>>(d);
     const int ntiles = sh.scan_tiles_l + sh.scan_tiles_h + sh.scan_tiles_g;
-    k_compact_reduce<<<ntiles, kScanThreads, 0, st>>>(d, sh, vals,
-                                                      d.list_g[par]);
-    k_compact_top<<<1, 1024, 0, st>>>(d, sh);
-    k_compact_scatter<<<ntiles, kScanThreads, 0, st>>>(
-        d, sh, vals, d.list_g[par], d.list_l[par ^ 1], d.list_h[par ^ 1],
-        d.list_g[par ^ 1]);
-    mark(7);
-    k_finalize<<<sh.S, 256, 0, st>>>(d);
+    auto end = [&](int nfin, int tiles) {
+        k_end_step<<<nfin + tiles, kScanThreads, 0, st>>>(d, sh, nfin, vals, d.list_g[par],
+                                                          d.list_l[par ^ 1], d.list_h[par ^ 1],
+                                                          d.list_g[par ^ 1]);
+    };
+    if (ev) {
+        end(0, ntiles);
+        mark(7);
+        end(sh.S, 0);
+    } else {
+        end(sh.S, ntiles);
+    }
     mark(8);
 }
 
@@ -2555,9 +2592,10 @@ void launch_frame_pack(const DevState& d, const int* list, int n, int lo, int hi
 
 int frame_tiles(int n) { return (n + kFrameTile - 1) / kFrameTile; }
 
-void launch_filter_scene(const DevState& d, const StepShape& sh, int scene,
+void launch_filter_scene(const DevState& base, const StepShape& sh, int scene,
                          int n_l, int n_h, int n_g, void* stream) {
     hipStream_t st = (hipStream_t)stream;
+    const DevState d = at_parity(base, sh.list_parity);
     const int par = sh.list_parity;
     const int ntiles = sh.scan_tiles_l + sh.scan_tiles_h + sh.scan_tiles_g;
     k_filter_count<<<ntiles, kScanThreads, 0, st>>>(d, sh, scene, d.list_l[par],
@@ -2568,9 +2606,10 @@ void launch_filter_scene(const DevState& d, const StepShape& sh, int scene,
         d.list_h[par ^ 1], d.list_g[par ^ 1], n_l, n_h, n_g);
 }
 
-void launch_work_counts(const DevState& d, const StepShape& sh,
+void launch_work_counts(const DevState& base, const StepShape& sh,
                         unsigned long long* out, void* stream) {
     hipStream_t st = (hipStream_t)stream;
+    const DevState d = at_parity(base, sh.list_parity);
     enqueue_grid(d, sh, st, 0);
     (void)hipMemsetAsync(out, 0, kWorkCounts * sizeof(unsigned long long), st);
     k_work<<<sh.grid_elem, 256, 0, st>>>(d, out);
@@ -2578,8 +2617,9 @@ void launch_work_counts(const DevState& d, const StepShape& sh,
 
 // Pair recording (tests): the grid of the current lists, then both levels'
 // density and force kernels in their recording variant.
-void launch_pair_record(const DevState& d, const StepShape& sh, void* stream) {
+void launch_pair_record(const DevState& base, const StepShape& sh, void* stream) {
     hipStream_t st = (hipStream_t)stream;
+    const DevState d = at_parity(base, sh.list_parity);
     const int cur = enqueue_grid(d, sh, st, 0);
     const uint32_t* vals = d.vals[cur];
     const uint32_t* keys = d.keys[cur];
@@ -2592,10 +2632,11 @@ void launch_pair_record(const DevState& d, const StepShape& sh, void* stream) {
 }
 
 // Neighbour inspection of the first n entries of a level's current list.
-void launch_neighbors_n(const DevState& d, const StepShape& sh, int scene,
+void launch_neighbors_n(const DevState& base, const StepShape& sh, int scene,
                         int level, int n, uint32_t* counts, uint32_t* sums,
                         void* stream) {
     hipStream_t st = (hipStream_t)stream;
+    const DevState d = at_parity(base, sh.list_parity);
     const int cur = enqueue_grid(d, sh, st, 1);
     const int par = sh.list_parity;
     const int* list = level ? d.list_h[par] : d.list_l[par];
