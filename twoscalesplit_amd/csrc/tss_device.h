@@ -62,7 +62,8 @@ constexpr int kRedFields = 9;
 struct SceneDev {
     // geometry
     float ox, oy;             // domain origin
-    float h, H;               // support radii (low / high)
+    float h, H;               // support radii (low / high), the cells' sizes
+    float inv_h, inv_H;       // their reciprocals, rounded (0: not usable)
     int dlx, dly, dhx, dhy;   // grid dimensions
     int cbase_l, cbase_h;     // unified cell bases
     int lbase, lcap;          // low ids owned

@@ -603,6 +603,11 @@ struct tss_batch {
         s.oy = c.domain_origin[1];
         s.h = c.effective_radius;
         s.H = c.effective_radius_high;
+        // the device's quotient by reciprocal is exact where nothing of it
+        // leaves the normal range (axis_cell)
+        auto reciprocal = [](float x) { return x > 1e-18f && x < 1e18f ? 1.0f / x : 0.0f; };
+        s.inv_h = reciprocal(s.h);
+        s.inv_H = reciprocal(s.H);
         s.dlx = c.domain_dims[0];
         s.dly = c.domain_dims[1];
         s.dhx = c.domain_dims_high[0];

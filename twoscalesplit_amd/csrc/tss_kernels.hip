@@ -33,9 +33,26 @@ constexpr uint8_t kActive = 0, kTransient = 1, kDeleted = 2;
 
 // Grid coordinate along one axis: clamp((int)(((x+off)-o)/cell), 0, dim-1)
 // (R:241-289); the clamp is taken in float so every input is defined.
+// inv = 1 / cell rounded: the quotient is the product with inv, corrected
+// twice by its exact residual (Markstein's division: a faithful quotient,
+// then the correctly rounded one), 5 instructions against the division's 11.
+// An overflowing product is kept as it is (the residual would be NaN), and
+// inv = 0 asks for the division (cells of extreme size). Eight such quotients
+// are a target's set-up in each neighbour kernel, which instructions bound:
+// with row_run below, density<low> 103 -> 99.8 and density<high> 333 -> 327 us
+// at 200k + 200k targets.
 __device__ __forceinline__ int axis_cell(float x, float off, float o,
-                                         float cell, int dim) {
-    float t = ((x + off) - o) / cell;
+                                         float cell, float inv, int dim) {
+    const float a = (x + off) - o;
+    float t;
+    if (__builtin_expect(inv != 0.0f, 1)) {
+        const float q = a * inv;
+        t = fmaf(fmaf(-cell, q, a), inv, q);
+        t = fmaf(fmaf(-cell, t, a), inv, t);
+        t = q < 1e9f ? t : q;
+    } else {
+        t = a / cell;
+    }
     if (!(t >= 1.0f)) return 0;
     if (t >= (float)dim) return dim - 1;
     return (int)t;
@@ -102,40 +119,54 @@ struct Box {
 __device__ __forceinline__ Box scan_box(const SceneDev& sc, bool high, float2 x,
                                         float r) {
     const float cell = high ? sc.H : sc.h;
+    const float inv = high ? sc.inv_H : sc.inv_h;
     const int dx = high ? sc.dhx : sc.dlx;
     const int dy = high ? sc.dhy : sc.dly;
     Box b;
-    b.x0 = axis_cell(x.x, -r, sc.ox, cell, dx);
-    b.x1 = axis_cell(x.x, r, sc.ox, cell, dx);
-    b.y0 = axis_cell(x.y, -r, sc.oy, cell, dy);
-    b.y1 = axis_cell(x.y, r, sc.oy, cell, dy);
+    b.x0 = axis_cell(x.x, -r, sc.ox, cell, inv, dx);
+    b.x1 = axis_cell(x.x, r, sc.ox, cell, inv, dx);
+    b.y0 = axis_cell(x.y, -r, sc.oy, cell, inv, dy);
+    b.y1 = axis_cell(x.y, r, sc.oy, cell, inv, dy);
     return b;
 }
 
 // Contiguous sorted range covering cells x0..x1 of one grid row (cells are
-// row-major, so neighbouring cells of a row are adjacent in sorted order).
-// The entries of four cells are loaded together, then combined in order.
+// row-major, so neighbouring cells of a row are adjacent in sorted order):
+// from the first non-empty cell's start to the last one's end, (-1, -1) if
+// all are empty. Starts and ends rise along a row and an empty cell holds -1,
+// so these are the least start (unsigned) and the greatest end. Four cells
+// are loaded together (a same-level row spans at most four; indices clamped
+// into the row: a repeated cell changes neither). need0: only cells that hold
+// a state-0 particle.
+template <bool NEED = false>
 __device__ __forceinline__ void row_run(const int* __restrict__ cs,
                                         const int* __restrict__ ce, int row,
-                                        int x0, int x1, int& s, int& e) {
-    s = -1;
-    e = -1;
-    for (int c0 = x0; c0 <= x1; c0 += 4) {
-        int st[4], en[4];
+                                        int x0, int x1, int& s, int& e,
+                                        const uint8_t* __restrict__ cf = nullptr,
+                                        bool need0 = false) {
+    uint32_t lo = ~0u;
+    int hi = -1;
+    auto four = [&](int c0) {
+        uint32_t st[4];
+        int en[4];
+        uint8_t f[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const int cx = row + min(c0 + k, x1);
-            st[k] = cs[cx];
-            en[k] = ce[cx];
+            const uint32_t cx = (uint32_t)(row + min(c0 + k, x1));
+            st[k] = (uint32_t)gather(cs, cx);
+            en[k] = gather(ce, cx);
+            if (NEED) f[k] = need0 ? gather(cf, 2u * cx) : (uint8_t)1;
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            if (c0 + k <= x1 && st[k] >= 0) {
-                if (s < 0) s = st[k];
-                e = en[k];
-            }
+            lo = min(lo, NEED && !f[k] ? ~0u : st[k]);
+            hi = max(hi, NEED && !f[k] ? -1 : en[k]);
         }
-    }
+    };
+    four(x0);
+    for (int c0 = x0 + 4; c0 <= x1; c0 += 4) four(c0);
+    s = (int)lo;
+    e = hi;
 }
 
 // Blended M4 kernel (R:116-239, 358-361): W_bar = (W_h + W_H)/2 and the
@@ -379,12 +410,12 @@ __global__ void k_begin_hash(DevState d, int nclear, int count, int solo, int nt
             const SceneDev& sc = d.scenes[s];
             const float2 x = d.pos[u];
             if (!high) {
-                int cx = axis_cell(x.x, 0.0f, sc.ox, sc.h, sc.dlx);
-                int cy = axis_cell(x.y, 0.0f, sc.oy, sc.h, sc.dly);
+                int cx = axis_cell(x.x, 0.0f, sc.ox, sc.h, sc.inv_h, sc.dlx);
+                int cy = axis_cell(x.y, 0.0f, sc.oy, sc.h, sc.inv_h, sc.dly);
                 key = (uint32_t)(sc.cbase_l + cy * sc.dlx + cx);
             } else {
-                int cx = axis_cell(x.x, 0.0f, sc.ox, sc.H, sc.dhx);
-                int cy = axis_cell(x.y, 0.0f, sc.oy, sc.H, sc.dhy);
+                int cx = axis_cell(x.x, 0.0f, sc.ox, sc.H, sc.inv_H, sc.dhx);
+                int cy = axis_cell(x.y, 0.0f, sc.oy, sc.H, sc.inv_H, sc.dhy);
                 key = (uint32_t)(sc.cbase_h + cy * sc.dhx + cx);
             }
             keys[k] = key;
