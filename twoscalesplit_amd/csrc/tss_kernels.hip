@@ -40,7 +40,7 @@ constexpr uint8_t kActive = 0, kTransient = 1, kDeleted = 2;
 // inv = 0 asks for the division (cells of extreme size). Eight such quotients
 // are a target's set-up in each neighbour kernel, which instructions bound:
 // with row_run below, density<low> 103 -> 99.8 and density<high> 333 -> 327 us
-// at 200k + 200k targets.
+// at 1M + 4M targets.
 __device__ __forceinline__ int axis_cell(float x, float off, float o,
                                          float cell, float inv, int dim) {
     const float a = (x + off) - o;
@@ -75,6 +75,12 @@ template <class T>
 __device__ __forceinline__ T gather(const T* __restrict__ base, uint32_t i) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) +
                                        (size_t)(i * (uint32_t)sizeof(T)));
+}
+
+// The element at byte offset o.
+template <class T>
+__device__ __forceinline__ T gather_byte(const T* __restrict__ base, uint32_t o) {
+    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (size_t)o);
 }
 
 // Element j + i through the 32-bit byte offset of j, i a small constant: the
