@@ -232,6 +232,17 @@ enum { kTuneDensityLow = 0, kTuneDensityHigh, kTuneForceLow, kTuneForceHigh,
 // lanes per target.
 constexpr long long kCoop8Targets = 16384;
 constexpr long long kCoop4Targets = 49152;
+// Low ids up to which both levels share a launch of the density and one of the
+// force (one lane per target, no phase timed): the levels' blocks run side by
+// side, where each alone leaves the chip partly idle. us per step with a
+// launch per level / shared, one scene alone (and three at once, on their
+// streams): half split 32k 150/105 (60/44), 100k 179/151 (89/80), 200k 242/208
+// (145/142), 400k 368/340 (279/284); all split 32k 147/103 (61/48), 100k
+// 205/168 (117/111), 200k 298/270 (215/211), 400k 500/471 (426/427); band rule
+// 64k 91/89 (38/37), 200k 112/107 (60/59), 400k 159/153 (104/108), 800k
+// 250/246 (198/212): once a level fills the chip, sharing only takes waves
+// from the other streams (the shared force runs 4 waves per SIMD, not 5).
+constexpr long long kBothLevelsCap = 262144;
 struct StepShape {
     int passes;               // radix passes
     int key_bits;

@@ -1911,7 +1911,10 @@ struct tss_batch {
         HIP_CHECK(hipStreamSynchronize(stream));
         if (!raw_ptr) {
             raw_ptr = true;
-            if (sh.copy_only) update_shape();
+            if (sh.copy_only) {
+                sh.copy_only = 0;
+                invalidate_graphs();
+            }
         }
         return v.dev;
     }

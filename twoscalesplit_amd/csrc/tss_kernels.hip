@@ -2563,16 +2563,24 @@ void launch_step(const DevState& base, const StepShape& sh, void* stream,
     else if (sh.coop == 4)
         launch_coop<4>(d, sh, vals, keys, st, ev == nullptr, mark);
     else {
-        launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
-        mark(2);
-        if (sh.two)
-            launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh], 4 * sh.cap_alive,
-                                     st);
+        const bool both = sh.two && !ev && sh.cap_alive <= kBothLevelsCap;
+        if (!both || !launch_both<false>(d, vals, keys, sh.tune[kTuneDensityLow],
+                                         sh.tune[kTuneDensityHigh], sh.cap_alive, st)) {
+            launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
+            mark(2);
+            if (sh.two)
+                launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh],
+                                         4 * sh.cap_alive, st);
+        }
         mark(3);
-        launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
-        mark(4);
-        if (sh.two)
-            launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive, st);
+        if (!both || !launch_both<true>(d, vals, keys, sh.tune[kTuneForceLow],
+                                        sh.tune[kTuneForceHigh], sh.cap_alive, st)) {
+            launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
+            mark(4);
+            if (sh.two)
+                launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive,
+                                        st);
+        }
     }
     mark(5);
     // the reductions, split candidates and groups in one launch (two where
