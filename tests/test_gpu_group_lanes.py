@@ -46,7 +46,7 @@ def _scene(kind):
 @pytest.mark.parametrize("expected", [16384, 49152])
 def test_lanes_per_target_do_not_change_results(kind, expected):
     sc = _scene(kind)
-    cap = expected // (2 if sc.cfg.mode == MODE_REFERENCE else 1)
+    cap = expected // (3 if sc.cfg.mode == MODE_REFERENCE else 1)
     print("[case]", kind, expected, flush=True)
     a = Solver(sc.cfg, sc.low_xy, cap, sc.bnd_xy)
     b = Solver(sc.cfg, sc.low_xy, cap, sc.bnd_xy)

@@ -525,16 +525,18 @@ struct tss_batch {
         for (int k = 0; k < tss::kPairKernels; ++k) sh.tune[k] = tune[k];
         // several lanes per target where one per target leaves the chip idle
         // (and no launch shape was set by the caller), by the targets to
-        // expect: every low particle, twice as many under the reference
+        // expect: every low particle, three times as many under the reference
         // rule. us per step with 1 / 4 / 8 lanes per target, one scene alone
-        // (and three at once, on their streams): plain 8k 114/84/77
-        // (41/31/29), 32k 115/89/90 (44/37/40), 48k 115/93/97 (46/44/46), 64k
-        // 118/104/110 (48/51/66); half split 8k 181/97/93 (65/38/39), 24k
-        // 189/120/131 (74/62/79), 32k 191/134/156 (75/74/97); all split 8k
-        // 167/98/100 (62/41/44), 24k 184/142/160 (73/72/93)
+        // (and three at once, on their streams): plain 8k 82/-/54
+        // (30/-/21), 16k 83/-/57 (30/-/23), 32k 84/66/- (32/28/-), 48k
+        // 84/72/- (34/34/-), 64k 86/104/- (35/51/-); half split 4k 94/-/62
+        // (34/-/24), 8k 98/71/68 (36/29/30), 16k 96/78/- (38/37/-), 20k
+        // 98/89/- (40/46/-), 24k 105/95/- (43/51/-); all split 4k 83/-/61
+        // (30/-/24), 8k 85/73/74 (33/31/35), 12k 87/82/- (35/39/-), 16k 91/93/- (37/48/-), 20k
+        // 93/105/- (39/58/-)
         long long expect = 0;
         for (const SceneHost& s : scenes)
-            if (s.alive) expect += (s.cfg.mode == TSS_MODE_REFERENCE ? 2LL : 1LL) * s.lcap;
+            if (s.alive) expect += (s.cfg.mode == TSS_MODE_REFERENCE ? 3LL : 1LL) * s.lcap;
         sh.coop = shapes_set || expect > tss::kCoop4Targets ? 0
                   : expect > tss::kCoop8Targets             ? 4
                                                             : 8;
