@@ -2,7 +2,8 @@
 target, the levels' launch shapes equal) against a launch per level (shapes
 that differ): the same bits, from the first step (no high particle) on, with
 counts around a block's, one scene and several, and past the capacity up to
-which a launch is shared.
+which a launch is shared. A batch with a band-rule scene cuts the high level's
+blocks to 262144 targets: with more, a scene is what it is alone.
 """
 from __future__ import annotations
 
@@ -60,3 +61,24 @@ def test_several_scenes():
             b.close()
     for x, y in zip(*out):
         np.testing.assert_array_equal(x, y)
+
+
+def test_more_high_targets_than_blocks_of_a_band_batch():
+    big = scenes.small_two_scale(nx=280, ny=250, nxd=300, nyd=260, mode=MODE_REFERENCE,
+                                 split_x=-1.0)
+    band = scenes.small_two_scale(nx=24, ny=30, mode=MODE_BAND)
+    scs = (big, band)
+    b = Batch(2, sum(len(s.low_xy) for s in scs), sum(len(s.bnd_xy) for s in scs),
+              sum(s.cells[0] for s in scs), sum(s.cells[1] for s in scs))
+    a = Solver(big.cfg, big.low_xy, len(big.low_xy), big.bnd_xy)
+    try:
+        ids = [b.add_scene(s.cfg, s.low_xy, len(s.low_xy), s.bnd_xy) for s in scs]
+        for steps in (2, 3):
+            a.step_graph(steps)
+            b.step_graph(steps)
+        assert a.counts()["n_high"] == 280000
+        for f in ("POS_H", "VEL_H", "RHO_H", "POS_L", "VEL_L", "RHO_L"):
+            np.testing.assert_array_equal(a.read(f), b.read(ids[0], f), err_msg=f)
+    finally:
+        a.close()
+        b.close()

@@ -238,10 +238,14 @@ constexpr long long kCoop4Targets = 49152;
 // launch per level / shared, one scene alone (and three at once, on their
 // streams): half split 32k 150/105 (60/44), 100k 179/151 (89/80), 200k 242/208
 // (145/142), 400k 368/340 (279/284); all split 32k 147/103 (61/48), 100k
-// 205/168 (117/111), 200k 298/270 (215/211), 400k 500/471 (426/427); band rule
-// 64k 91/89 (38/37), 200k 112/107 (60/59), 400k 159/153 (104/108), 800k
-// 250/246 (198/212): once a level fills the chip, sharing only takes waves
-// from the other streams (the shared force runs 4 waves per SIMD, not 5).
+// 205/168 (117/111), 200k 298/270 (215/211), 400k 500/471 (426/427): once each
+// level fills the chip, sharing only takes waves from the other streams (the
+// shared force runs 4 waves per SIMD, not 5). Under the band rule the density
+// always shares (its few high targets, which wait on their gathers, run beside
+// the low ones): 400k 156/154 (102/101), 1M 294/292 (243/241), 64 scenes of
+// 2k to 64k with 50k high particles 507/485 (351/347); the force as above
+// (both shared: 1M 293 (243), and 505 us for two steps of it on launch shapes
+// set for large scenes against 492).
 constexpr long long kBothLevelsCap = 262144;
 struct StepShape {
     int passes;               // radix passes

@@ -6,11 +6,11 @@
 // placement) rounds each operation exactly like the FP32 method definition;
 // the physics sums use explicit fmaf where a fused operation is wanted.
 //
-// Step (one launch per phase for all scenes of a batch):
-//   fill -> hash -> radix sort (P passes x {hist, scan, scatter})
-//   -> ranges+reorder -> density -> force+integrate -> reduce
-//   -> split candidates -> groups -> cap -> compaction (3 kernels)
-//   -> finalize
+// Step (for all scenes of a batch):
+//   clear + hash -> counting sort by cell (or a radix sort) -> reorder
+//   -> density -> force + integrate (both levels in a launch, or one each)
+//   -> reductions, split candidates and groups in a launch -> cap
+//   -> compaction and finalize in a launch
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -2563,23 +2563,24 @@ void launch_step(const DevState& base, const StepShape& sh, void* stream,
     else if (sh.coop == 4)
         launch_coop<4>(d, sh, vals, keys, st, ev == nullptr, mark);
     else {
-        const bool both = sh.two && !ev && sh.cap_alive <= kBothLevelsCap;
-        if (!both || !launch_both<false>(d, vals, keys, sh.tune[kTuneDensityLow],
-                                         sh.tune[kTuneDensityHigh], sh.cap_alive, st)) {
+        const bool force_both = sh.two && !ev && sh.cap_alive <= kBothLevelsCap;
+        const bool density_both = force_both || (sh.band_any && !ev);
+        if (!density_both || !launch_both<false>(d, vals, keys, sh.tune[kTuneDensityLow],
+                                         sh.tune[kTuneDensityHigh], sh.cap_alive, sh.band_any, st)) {
             launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
             mark(2);
             if (sh.two)
                 launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh],
-                                         4 * sh.cap_alive, st);
+                                         4 * sh.cap_alive, st, sh.band_any);
         }
         mark(3);
-        if (!both || !launch_both<true>(d, vals, keys, sh.tune[kTuneForceLow],
-                                        sh.tune[kTuneForceHigh], sh.cap_alive, st)) {
+        if (!force_both || !launch_both<true>(d, vals, keys, sh.tune[kTuneForceLow],
+                                        sh.tune[kTuneForceHigh], sh.cap_alive, sh.band_any, st)) {
             launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
             mark(4);
             if (sh.two)
                 launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive,
-                                        st);
+                                        st, sh.band_any);
         }
     }
     mark(5);
