@@ -243,8 +243,10 @@ int tss_work_counts(tss_solver* s, unsigned long long out[TSS_WORK_COUNT]);
  * targets, [1] density high, [2] force low, [3] force high. block: 128, 256
  * or 512 threads; depth: LDS buffer depth, 8, 16 or 32 pairs per lane;
  * xcd_order: 1 gives each of the 8 XCDs one contiguous range of blocks;
- * grid: 0 = one thread per target of capacity, else a persistent grid of at
- * most this many blocks. Results never depend on the shapes (every
+ * grid: 0 = one thread per target of capacity (high targets of a batch with a
+ * band-rule scene: of 262144 at most), else a persistent grid of at
+ * most this many blocks. Equal block and depth of both levels let them share
+ * a launch on batches of up to 262144 low ids. Results never depend on the shapes (every
  * neighbour sum is lane-local). Default: 256, 16, 0, 0. No counterpart in
  * the reference (fixed 256-thread blocks, R/WCSPHSolver.cu:2421). */
 typedef struct tss_tuning {

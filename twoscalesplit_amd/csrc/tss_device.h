@@ -227,7 +227,6 @@ struct PairTune {
 enum { kTuneDensityLow = 0, kTuneDensityHigh, kTuneForceLow, kTuneForceHigh,
        kPairKernels };
 
-// Host-known launch parameters of one step.
 // Expected targets up to which a batch's neighbour sums take eight (four)
 // lanes per target.
 constexpr long long kCoop8Targets = 16384;
@@ -247,6 +246,8 @@ constexpr long long kCoop4Targets = 49152;
 // (both shared: 1M 293 (243), and 505 us for two steps of it on launch shapes
 // set for large scenes against 492).
 constexpr long long kBothLevelsCap = 262144;
+
+// Host-known launch parameters of one step.
 struct StepShape {
     int passes;               // radix passes
     int key_bits;

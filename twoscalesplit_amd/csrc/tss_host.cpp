@@ -499,9 +499,10 @@ struct tss_batch {
         sh.key_cells = (int)maxkey;
         sh.cell_tiles = (int)((maxkey + tss::kCellTile - 1) / tss::kCellTile);
         // the grid build's sort: the counting sort where the resident cells
-        // number at most kCountCellsPerKey per key (five short launches,
-        // faster than the one-workgroup radix sort even on small batches:
-        // 0.104 vs 0.128 ms per C1/C2 step), else the one-workgroup radix
+        // number at most kCountCellsPerKey per key (four or five short
+        // launches, faster than the one-workgroup radix sort even on small
+        // batches: 0.104 vs 0.128 ms per step of 8k particles with the
+        // other launches as they were then), else the one-workgroup radix
         // sort where the keys fit, else the multi-tile radix sort; a forced
         // one-workgroup sort that no longer fits (scenes added since) falls
         // back to this choice
