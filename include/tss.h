@@ -209,8 +209,8 @@ int tss_neighbors(tss_solver* s, int level, uint32_t* counts, uint32_t* sums,
  * of tss_neighbors restricted to nonzero state weights: [0] same-level
  * density, [1] cross-level density, [2] same-level force, [3] cross-level
  * force, [4] wall candidates of the force. The kernels run on the current
- * state in a recording variant -- the same candidate masks, scans and row
- * and pass skips as a step -- after a grid build of the current lists; no
+ * state in a recording variant -- the same lanes per target, candidate
+ * masks, scans and row and pass skips as a step -- after a grid build of the current lists; no
  * state is advanced (relaxation sub-steps are not run). These are the sets
  * of updateDensityCell* (R/WCSPHSolver.cu:335-474) and updateAccCell*
  * (R/WCSPHSolver.cu:476-885) with their lambda tables; no counterpart

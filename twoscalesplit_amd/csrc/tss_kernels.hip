@@ -2662,13 +2662,18 @@ void launch_work_counts(const DevState& base, const StepShape& sh,
 }
 
 // Pair recording (tests): the grid of the current lists, then both levels'
-// density and force kernels in their recording variant.
+// density and force kernels, with the step's lanes per target, in their
+// recording variant.
 void launch_pair_record(const DevState& base, const StepShape& sh, void* stream) {
     hipStream_t st = (hipStream_t)stream;
     const DevState d = at_parity(base, sh.list_parity);
     const int cur = enqueue_grid(d, sh, st, 0);
     const uint32_t* vals = d.vals[cur];
     const uint32_t* keys = d.keys[cur];
+    if (sh.coop == 8)
+        return launch_coop<8, true>(d, sh, vals, keys, st, true, [](int) {});
+    if (sh.coop == 4)
+        return launch_coop<4, true>(d, sh, vals, keys, st, true, [](int) {});
     const int gl = blocks_for(sh.cap_alive, 256, 16384);
     const int gh = blocks_for(4 * sh.cap_alive, 256, 16384);
     k_density<false, 256, 16, true><<<gl, 256, 0, st>>>(d, vals, keys, 0);
