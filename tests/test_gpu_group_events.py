@@ -1,0 +1,82 @@
+"""Groups that are promoted, merged back or dissolved, counted per wave: many
+small scenes whose groups share waves and compaction tiles take the steps that
+each takes alone; and a step that dissolves the surface's groups is not much
+longer than one that changes nothing.
+"""
+from __future__ import annotations
+
+import time
+
+import numpy as np
+import pytest
+
+from twoscalesplit_amd import MODE_BAND, MODE_REFERENCE, Batch, Solver, scenes
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = ("n_low", "n_high", "n_groups", "n_split", "n_promote", "n_merge", "n_dissolve")
+
+
+@pytest.mark.parametrize("promote", [0, 2])
+def test_scenes_together_and_alone(promote):
+    rng = np.random.default_rng(promote)
+    scs = []
+    for i in range(24):
+        sc = scenes.small_two_scale(seed=i, nx=int(rng.integers(1, 20)), ny=int(rng.integers(1, 16)),
+                                    mode=MODE_REFERENCE if i % 7 == 3 else MODE_BAND,
+                                    split_x=0.02)
+        if promote:
+            sc.cfg.promote_min_age, sc.cfg.promote_max_age = promote, 2 * promote
+        # some scenes sink into their walls' corner: their surface moves
+        sc.low_xy = (sc.low_xy * np.float32(rng.uniform(0.8, 1.1))).astype(np.float32)
+        scs.append(sc)
+    print("[case]", promote, flush=True)
+    b = Batch(len(scs), sum(len(s.low_xy) for s in scs), sum(len(s.bnd_xy) for s in scs),
+              sum(s.cells[0] for s in scs), sum(s.cells[1] for s in scs))
+    alone = [Solver(s.cfg, s.low_xy, len(s.low_xy), s.bnd_xy) for s in scs]
+    seen = dict.fromkeys(COUNTS, 0)
+    try:
+        ids = [b.add_scene(s.cfg, s.low_xy, len(s.low_xy), s.bnd_xy) for s in scs]
+        for _ in range(30):
+            b.step(1)
+            for i, a in zip(ids, alone):
+                a.step(1)
+                ca, cb = a.counts(), b.counts(i)
+                assert {k: ca[k] for k in COUNTS} == {k: cb[k] for k in COUNTS}
+                for k in COUNTS:
+                    seen[k] += ca[k]
+        for i, a in zip(ids, alone):
+            for f in ("LIST_L", "LIST_H", "LIST_G", "STATE_L", "STATE_H", "POS_L", "POS_H"):
+                np.testing.assert_array_equal(a.read(f), b.read(i, f), err_msg=f)
+    finally:
+        b.close()
+        for a in alone:
+            a.close()
+    print("[seen]", seen, flush=True)
+    assert seen["n_split"] > 0 and seen["n_dissolve"] > 0
+    assert not promote or (seen["n_promote"] > 0 and seen["n_merge"] > 0)
+
+
+def test_dissolving_a_surface_costs_little():
+    """With an atomic per entry such a step took 2.9 times a calm one."""
+    dissolve = calm = np.inf
+    for seed in range(3):
+        sc = scenes.c3_large(seed=seed, forced=False)
+        sol = Solver(sc.cfg, sc.low_xy, sc.cap_low, sc.bnd_xy)
+        try:
+            sol.step(3)
+            for _ in range(16):
+                sol.synchronize()
+                t = time.perf_counter()
+                sol.step(1)
+                sol.synchronize()
+                t = time.perf_counter() - t
+                c = sol.counts()
+                if c["n_dissolve"] > 5000:
+                    dissolve = min(dissolve, t)
+                elif c["n_dissolve"] + c["n_split"] == 0:
+                    calm = min(calm, t)
+        finally:
+            sol.close()
+    print("[us]", dissolve * 1e6, calm * 1e6, flush=True)
+    assert dissolve < 1.6 * calm

@@ -1446,16 +1446,33 @@ __device__ __forceinline__ float2 clamp_child(float2 ph, float2 pl, double rmax)
     return make_float2(pl.x + ox, pl.y + oy);
 }
 
+// f(key, number of lanes with it) once per distinct key of the lanes that are
+// on, on the first of them.
+template <class F>
+__device__ __forceinline__ void per_key(bool on, int key, F f) {
+    uint64_t todo = __ballot(on);
+    while (todo != 0ull) {
+        const int first = __ffsll((long long)todo) - 1;
+        const int key0 = __shfl(key, first, 64);
+        const uint64_t same = __ballot(on && key == key0) & todo;
+        if ((int)(threadIdx.x & 63) == first) f(key, (int)__popcll(same));
+        todo &= ~same;
+    }
+}
+
 // Existing groups: age, promotion (dormant test of R:1053-1095, enabled by
 // the method), child clamp (R:1097-1172), merge decision and application.
 // LANES lanes per group: under the band rule the merge test scans the
 // neighbourhoods of up to four children, one child per lane; the lanes of a
 // group sit in one wave and OR their results in a ballot, and lane 0
 // applies the decision. LANES = 1 tests the children in turn.
-// Entries that leave the lists here are counted per scene and compaction
-// tile (sidx is written where a band rule can remove any). th, tg: the first
-// compaction tile of the high and the group lists. thread, nthreads: of this
-// part of the launch.
+// Entries that leave the lists here (under the band rule only, which takes
+// four lanes; sidx is written where one is resident) are counted per scene and
+// compaction tile, by one atomic per wave and distinct scene or tile: a step
+// that dissolves the surface's groups (10,600 at a million low ids) otherwise
+// waits on a few counters (that step 900 us with an atomic per entry, 377 us
+// so). th, tg: the first compaction tile of the high and the group lists.
+// thread, nthreads: of this part of the launch.
 template <int LANES>
 __device__ __forceinline__ void update_groups(const DevState& d, const uint32_t* __restrict__ vals,
                                               const int* __restrict__ list_g, int solo, int th, int tg, int thread,
@@ -1497,78 +1514,81 @@ __device__ __forceinline__ void update_groups(const DevState& d, const uint32_t*
             const uint64_t bal = __ballot(mine);
             const int g0 = (threadIdx.x & 63) & ~(LANES - 1);
             keep = ((bal >> g0) & ((1ull << LANES) - 1ull)) != 0ull;
-            if (kl != 0) continue;
         }
         // merged: 1 = promoted group merged back (parent re-listed),
         //         2 = transient group dissolved (parent already listed)
         uint8_t merged = 0;
-        if (st == kTransient) {
-            d.age[p] = age;
-            if (promote) {
-                d.state[p] = kDeleted;
-                for (int k = 0; k < 4; ++k) d.state[c0 + k] = 0;
-                atomicAdd(&d.scnt[s].n_promote, 1);
-                d.counts->events = 1;
-                // the parent leaves the low list (one that the list holds as
-                // deleted already is counted with the split candidates)
-                const uint32_t k = (uint32_t)d.sidx[p];
-                if (k < (uint32_t)nl && (int)vals[k] == p && d.sstate[k] != kDeleted) {
-                    atomicAdd(&d.tile_cnt[k / kScanTile].x, 1);
-                    atomicAdd(&d.scnt[s].drop_l, 1);
+        bool promoted = false;
+        if (kl == 0) {
+            if (st == kTransient) {
+                d.age[p] = age;
+                if (promote) {
+                    promoted = true;
+                    d.state[p] = kDeleted;
+                    for (int k = 0; k < 4; ++k) d.state[c0 + k] = 0;
+                } else if (sc.mode == 2 && !keep) {
+                    // dissolve: children leave the lists, the parent stays
+                    merged = 2;
+                    d.state[p] = kActive;
+                    d.age[p] = 0;
+                } else {
+                    const float2 pl = d.pos[p];
+                    const double rmax = clamp_radius(sc.m_l, d.rho[p]);
+                    float2 ph[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) ph[k] = d.pos[c0 + k];
+                    // stored only where the clamp changes a bit (within the
+                    // radius it returns the position itself, as a rule)
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float2 c = clamp_child(ph[k], pl, rmax);
+                        if (__float_as_uint(c.x) != __float_as_uint(ph[k].x) ||
+                            __float_as_uint(c.y) != __float_as_uint(ph[k].y))
+                            d.pos[c0 + k] = c;
+                    }
                 }
-            } else if (sc.mode == 2 && !keep) {
-                // dissolve: children leave the lists, the parent stays
-                merged = 2;
+            } else if (st == kDeleted && sc.mode == 2 && !keep) {
+                merged = 1;
+                float2 c[4], v[4];
+                for (int k = 0; k < 4; ++k) {
+                    c[k] = d.pos[c0 + k];
+                    v[k] = d.vel[c0 + k];
+                }
+                d.pos[p] = make_float2(((c[0].x + c[1].x) + (c[2].x + c[3].x)) * 0.25f,
+                                       ((c[0].y + c[1].y) + (c[2].y + c[3].y)) * 0.25f);
+                d.vel[p] = make_float2(((v[0].x + v[1].x) + (v[2].x + v[3].x)) * 0.25f,
+                                       ((v[0].y + v[1].y) + (v[2].y + v[3].y)) * 0.25f);
                 d.state[p] = kActive;
                 d.age[p] = 0;
-                atomicAdd(&d.scnt[s].n_dissolve, 1);
-                d.counts->events = 1;
-            } else {
-                const float2 pl = d.pos[p];
-                const double rmax = clamp_radius(sc.m_l, d.rho[p]);
-                float2 ph[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) ph[k] = d.pos[c0 + k];
-                // stored only where the clamp changes a bit (within the
-                // radius it returns the position itself, as a rule)
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float2 c = clamp_child(ph[k], pl, rmax);
-                    if (__float_as_uint(c.x) != __float_as_uint(ph[k].x) ||
-                        __float_as_uint(c.y) != __float_as_uint(ph[k].y))
-                        d.pos[c0 + k] = c;
-                }
+                for (int k = 0; k < 4; ++k) d.state[c0 + k] = 1;
             }
-        } else if (st == kDeleted && sc.mode == 2 && !keep) {
-            merged = 1;
-            float2 c[4], v[4];
-            for (int k = 0; k < 4; ++k) {
-                c[k] = d.pos[c0 + k];
-                v[k] = d.vel[c0 + k];
-            }
-            d.pos[p] = make_float2(((c[0].x + c[1].x) + (c[2].x + c[3].x)) * 0.25f,
-                                   ((c[0].y + c[1].y) + (c[2].y + c[3].y)) * 0.25f);
-            d.vel[p] = make_float2(((v[0].x + v[1].x) + (v[2].x + v[3].x)) * 0.25f,
-                                   ((v[0].y + v[1].y) + (v[2].y + v[3].y)) * 0.25f);
-            d.state[p] = kActive;
-            d.age[p] = 0;
-            for (int k = 0; k < 4; ++k) d.state[c0 + k] = 1;
-            atomicAdd(&d.scnt[s].n_merge, 1);
-            d.counts->events = 1;
+            d.merged[p] = merged;
         }
-        d.merged[p] = merged;
-        if (merged) {
-            // the group and its listed children leave the lists
-            int2& t = d.tile_cnt[tg + q / kScanTile];
-            atomicAdd(&t.x, 1);
-            if (merged == 1) atomicAdd(&t.y, 1);
-            for (int c = 0; c < 4; ++c) {
-                const uint32_t k = (uint32_t)d.sidx[c0 + c] - (uint32_t)nl;
-                if (k < (uint32_t)nh && (int)vals[nl + k] == c0 + c) {
-                    atomicAdd(&d.tile_cnt[th + k / kScanTile].x, 1);
-                    atomicAdd(&d.scnt[s].drop_h, 1);
-                }
-            }
+        if constexpr (LANES == 4) {
+            if (__ballot(promoted || merged != 0) == 0ull) continue;
+            d.counts->events = 1;
+            SceneCount* scnt = d.scnt;
+            int2* tiles = d.tile_cnt;
+            per_key(promoted, s, [&](int x, int n) { atomicAdd(&scnt[x].n_promote, n); });
+            per_key(merged == 1, s, [&](int x, int n) { atomicAdd(&scnt[x].n_merge, n); });
+            per_key(merged == 2, s, [&](int x, int n) { atomicAdd(&scnt[x].n_dissolve, n); });
+            // a promoted parent leaves the low list (one that the list holds
+            // as deleted already is counted with the split candidates)
+            uint32_t k = promoted ? (uint32_t)d.sidx[p] : ~0u;
+            const bool low = k < (uint32_t)nl && (int)vals[k] == p && d.sstate[k] != kDeleted;
+            per_key(low, (int)(k / kScanTile), [&](int x, int n) { atomicAdd(&tiles[x].x, n); });
+            per_key(low, s, [&](int x, int n) { atomicAdd(&scnt[x].drop_l, n); });
+            // a merged group and its listed children (one per lane) leave theirs
+            per_key(merged != 0, tg + q / kScanTile,
+                    [&](int x, int n) { atomicAdd(&tiles[x].x, n); });
+            per_key(merged == 1, tg + q / kScanTile,
+                    [&](int x, int n) { atomicAdd(&tiles[x].y, n); });
+            const bool gone = __shfl((int)merged, (int)(threadIdx.x & 63) & ~3, 64) != 0;
+            k = gone ? (uint32_t)d.sidx[c0 + kl] - (uint32_t)nl : ~0u;
+            const bool high = k < (uint32_t)nh && (int)vals[nl + k] == c0 + kl;
+            per_key(high, th + (int)(k / kScanTile),
+                    [&](int x, int n) { atomicAdd(&tiles[x].x, n); });
+            per_key(high, s, [&](int x, int n) { atomicAdd(&scnt[x].drop_h, n); });
         }
     }
 }
