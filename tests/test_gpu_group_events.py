@@ -1,7 +1,8 @@
-"""Groups that are promoted, merged back or dissolved, counted per wave: many
-small scenes whose groups share waves and compaction tiles take the steps that
-each takes alone; and a step that dissolves the surface's groups is not much
-longer than one that changes nothing.
+"""Steps with many events. Groups that are promoted, merged back or dissolved,
+counted per wave: many small scenes whose groups share waves and compaction
+tiles take the steps that each takes alone. Splits under the cap. And steps that
+dissolve the surface's groups, or split every particle, are not much longer than
+steps without.
 """
 from __future__ import annotations
 
@@ -80,3 +81,55 @@ def test_dissolving_a_surface_costs_little():
             sol.close()
     print("[us]", dissolve * 1e6, calm * 1e6, flush=True)
     assert dissolve < 1.6 * calm
+
+
+def test_splits_of_capped_scenes_together():
+    """Splits of a step: the candidates that the scene's cap leaves, whether it
+    binds, is reached exactly or has room, in one batch and later on."""
+    scs, want = [], []
+    for cap, n in ((0, 35), (4, 35), (136, 35), (140, 35), (0, 1), (3, 7), (40, 700)):
+        sc = scenes.small_two_scale(nx=n if n < 50 else 28, ny=1 if n < 50 else 25, nxd=48,
+                                    mode=MODE_REFERENCE, split_x=-1.0)
+        sc.cfg.cap_high = cap
+        scs.append(sc)
+        # cap_high 0 stands for four per low particle
+        want.append(min(n, cap // 4) if cap else n)
+    b = Batch(len(scs), sum(len(s.low_xy) for s in scs), sum(len(s.bnd_xy) for s in scs),
+              sum(s.cells[0] for s in scs), sum(s.cells[1] for s in scs))
+    try:
+        ids = [b.add_scene(s.cfg, s.low_xy, len(s.low_xy), s.bnd_xy) for s in scs]
+        b.step(1)
+        c = [b.counts(i) for i in ids]
+        assert [x["n_split"] for x in c] == want
+        assert [x["n_high"] for x in c] == [4 * w for w in want]
+        assert [x["n_groups"] for x in c] == want
+        b.step_graph(2)
+        c = [b.counts(i) for i in ids]
+        assert [x["n_split"] for x in c] == [0] * len(scs)
+        assert [x["n_groups"] for x in c] == want
+    finally:
+        b.close()
+
+
+def test_splitting_all_costs_little():
+    """A step that splits every particle took 416 us more than one that splits
+    none with two atomics per wave on the scene's counters, 235 with one."""
+    us = {}
+    for split_x in (-1.0, 100.0):
+        best = np.inf
+        for seed in range(4):
+            sc = scenes.c3_large(seed=seed, forced=True)
+            sc.cfg.split_x = split_x
+            sol = Solver(sc.cfg, sc.low_xy, sc.cap_low, sc.bnd_xy)
+            try:
+                sol.synchronize()
+                t = time.perf_counter()
+                sol.step(1)
+                sol.synchronize()
+                best = min(best, time.perf_counter() - t)
+                assert sol.counts()["n_split"] == (sc.cap_low if split_x < 0 else 0)
+            finally:
+                sol.close()
+        us[split_x] = best * 1e6
+    print("[us]", us, flush=True)
+    assert us[-1.0] < us[100.0] + 320.0

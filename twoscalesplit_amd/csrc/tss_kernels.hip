@@ -1408,17 +1408,11 @@ __device__ __forceinline__ void split_candidates(const DevState& d, int block, i
             if (first) {
                 SceneCount& c = d.scnt[s0];
                 if (dm) atomicAdd(&c.drop_l, (int)__popcll(dm));
-                if (cm) {
-                    atomicAdd(&c.cand, (int)__popcll(cm));
-                    atomicAdd(&c.n_split, (int)__popcll(cm));
-                }
+                if (cm) atomicAdd(&c.cand, (int)__popcll(cm));
             }
         } else {
             if (drop) atomicAdd(&d.scnt[s].drop_l, 1);
-            if (cand) {
-                atomicAdd(&d.scnt[s].cand, 1);
-                atomicAdd(&d.scnt[s].n_split, 1);
-            }
+            if (cand) atomicAdd(&d.scnt[s].cand, 1);
         }
     }
 }
@@ -1618,6 +1612,12 @@ __global__ __launch_bounds__(256) void k_adapt(DevState d, const uint32_t* __res
     }
 }
 
+// Splits that a scene's cap on high particles leaves room for.
+__device__ __forceinline__ int splits_allowed(const SceneDev& sc, const SceneCount& c) {
+    const long long allowed = ((long long)sc.cap_h - 4LL * c.n_g) / 4;
+    return allowed < 0 ? 0 : (int)allowed;
+}
+
 // High-particle cap (spec): where a scene has more split candidates than
 // its cap allows, keep the first ones in sorted order. One block per scene;
 // exits at once when the cap does not bind.
@@ -1625,12 +1625,10 @@ __global__ __launch_bounds__(256) void k_cap(DevState d) {
     __shared__ int part[256];
     const int s = blockIdx.x;
     const SceneDev& sc = d.scenes[s];
-    SceneCount& c = d.scnt[s];
+    const SceneCount& c = d.scnt[s];
     if (!sc.alive) return;
-    const long long allowed_ll = ((long long)sc.cap_h - 4LL * c.n_g) / 4;
-    const int allowed = allowed_ll < 0 ? 0 : (int)allowed_ll;
+    const int allowed = splits_allowed(sc, c);
     if (c.cand <= allowed) return;
-    if (threadIdx.x == 0) c.n_split = allowed;
     int run = 0;
     for (int base = c.seg_l0; base < c.seg_l1; base += 256) {
         int k = base + threadIdx.x;
@@ -1921,7 +1919,9 @@ __device__ __forceinline__ void finalize_scene(const DevState& d, const StepShap
         c.n_l_last = c.seg_l1 - c.seg_l0;
         c.n_h_last = c.seg_h1 - c.seg_h0;
         c.psteps += (unsigned long long)(c.n_l_last + c.n_h_last);
-        // next lists: low = kept + merged; high = kept + 4 per split
+        // next lists: low = kept + merged; high = kept + 4 per split (the
+        // candidates that k_cap left)
+        c.n_split = shp.cap_binds ? min(c.cand, splits_allowed(sc, c)) : c.cand;
         c.n_l = c.n_l_last - c.drop_l + c.n_merge;
         c.n_h = c.n_h_last - c.drop_h + 4 * c.n_split;
         c.n_g = c.n_g + c.n_split - c.n_merge - c.n_dissolve;
