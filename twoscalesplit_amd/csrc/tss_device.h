@@ -45,6 +45,14 @@ constexpr int kCellDirect = 64;
 constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;  // entries per compaction tile
+// Each tile of the compaction sums the counts of all live ones (tile_totals):
+// up to kTileDirect launched tiles (1.4 million low ids of two levels) one by
+// one, beyond them by sums of kTileGroup tiles, for a launch more. us of a
+// step's adaptivity and compaction with events, one by one / by groups: all
+// split 1M low ids 65/61, 2M 113/97, 8M 605/345, 30M 5250/1306; half split 500k
+// 26/29, 1M 45/46, 2M 73/68, 8M 310/218.
+constexpr int kTileGroup = kScanThreads;
+constexpr int kTileDirect = 4096;
 // FP64 reductions: a scene's sorted particles are cut into chunks of
 // kRedChunk; a scene owns ceil(5 cap_low / kRedChunk) chunk slots (from its
 // own capacity, so the partition -- and every rounding -- is the same alone
@@ -198,6 +206,7 @@ struct DevState {
     uint8_t* merged;          // [CL] merged flag per low id
     // [max_scan_tiles] per compaction tile: entries not kept, P1 entries
     int2* tile_cnt;
+    int2* tile_sum;           // the same per kTileGroup tiles of a list
     double* red;              // [red_slots * kRedFields]
     int* red_scene;           // [red_slots] scene of each chunk slot (-1 none)
     int* red_base;            // [S] first chunk slot of each scene
@@ -259,6 +268,7 @@ struct StepShape {
     int sort_tiles;           // sort tiles allocated (row stride of hist)
     int sort_grid;            // sort tiles launched (<= sort_tiles)
     int scan_tiles_l, scan_tiles_h, scan_tiles_g;  // compaction tiles launched
+    int tile_groups;          // groups of them summed first, 0: none (tile_totals)
     PairTune tune[kPairKernels];
     int coop;                 // neighbour sums: 8 or 4 lanes per target, 0: one (PairTune)
     int S;

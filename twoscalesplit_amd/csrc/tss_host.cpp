@@ -355,6 +355,7 @@ struct tss_batch {
         const int nst = (int)((CL + tss::kScanTile - 1) / tss::kScanTile) * 2 +
                         (int)((4 * CL + tss::kScanTile - 1) / tss::kScanTile);
         d.tile_cnt = dalloc<int2>((size_t)nst, owned);
+        d.tile_sum = dalloc<int2>((size_t)nst / tss::kTileGroup + 3, owned);
         red_cap = (int)((U + tss::kRedChunk - 1) / tss::kRedChunk) + max_scenes + 1;
         d.red = dalloc<double>((size_t)red_cap * tss::kRedFields, owned);
         d.red_scene = dalloc<int>(red_cap, owned);
@@ -483,6 +484,11 @@ struct tss_batch {
         sh.scan_tiles_l = (int)((cap + tss::kScanTile - 1) / tss::kScanTile);
         sh.scan_tiles_h = sh.two ? (int)((4 * cap + tss::kScanTile - 1) / tss::kScanTile) : 0;
         sh.scan_tiles_g = sh.two ? sh.scan_tiles_l : 0;
+        auto groups = [](int tiles) { return (tiles + tss::kTileGroup - 1) / tss::kTileGroup; };
+        sh.tile_groups = sh.scan_tiles_l + sh.scan_tiles_h + sh.scan_tiles_g <= tss::kTileDirect
+                             ? 0
+                             : groups(sh.scan_tiles_l) + groups(sh.scan_tiles_h) +
+                                   groups(sh.scan_tiles_g);
         sh.cap_binds = 0;
         sh.band_any = 0;
         for (const SceneHost& s : scenes) {

@@ -1659,7 +1659,8 @@ __global__ __launch_bounds__(256) void k_cap(DevState d) {
 //   P0 = keep (low: not deleted; high: group not merged; group: not merged)
 //   P1 = low: split admitted; group: merged.
 // k_adapt (and k_cap) left each tile's counts of entries not kept and of P1
-// in tile_cnt; a block sums those of the tiles before its own.
+// in tile_cnt; a block sums those of the tiles before its own (of many tiles,
+// k_tile_sums those of each group first).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void tile_seg(const StepShape& sh, int tile,
                                          int& seg, int& t) {
@@ -1681,6 +1682,38 @@ __device__ __forceinline__ void tile_seg(const StepShape& sh, int tile,
 // ballots.
 constexpr int kScanWaves = kScanThreads / 64;
 
+__device__ __forceinline__ int tile_groups_of(int tiles) {
+    return (tiles + kTileGroup - 1) / kTileGroup;
+}
+
+// The counts of each group of kTileGroup tiles of a segment, a block each
+// (tiles past the live entries hold zero).
+__global__ __launch_bounds__(kScanThreads) void k_tile_sums(DevState d, StepShape sh) {
+    __shared__ int2 lds[kScanWaves];
+    static_assert(kTileGroup == kScanThreads, "a tile per thread");
+    if (!d.counts->events) return;  // the step's counts are not read
+    const int gl = tile_groups_of(sh.scan_tiles_l), gh = tile_groups_of(sh.scan_tiles_h);
+    const int b = (int)blockIdx.x;
+    const int seg = b < gl ? 0 : b < gl + gh ? 1 : 2;
+    const int tiles = seg == 0 ? sh.scan_tiles_l : seg == 1 ? sh.scan_tiles_h : sh.scan_tiles_g;
+    const int first = seg == 0 ? 0 : seg == 1 ? sh.scan_tiles_l : sh.scan_tiles_l + sh.scan_tiles_h;
+    const int q = (b - (seg == 0 ? 0 : seg == 1 ? gl : gl + gh)) * kTileGroup + (int)threadIdx.x;
+    int2 w = q < tiles ? d.tile_cnt[first + q] : make_int2(0, 0);
+    for (int off = 32; off > 0; off >>= 1) {
+        w.x += __shfl_xor(w.x, off, 64);
+        w.y += __shfl_xor(w.y, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int x = 1; x < kScanWaves; ++x) {
+            w.x += lds[x].x;
+            w.y += lds[x].y;
+        }
+        d.tile_sum[b] = w;
+    }
+}
+
 // P0 and P1 totals of the segments, and of the tiles of segment `seg` before
 // its tile `t`; the same on every thread. lds: 7 ints per wave.
 struct TileTotals {
@@ -1695,18 +1728,35 @@ __device__ __forceinline__ TileTotals tile_totals(const DevState& d, const StepS
     const int first[3] = {0, sh.scan_tiles_l, sh.scan_tiles_l + sh.scan_tiles_h};
     // entries not kept, P1 (high tiles have none), and both before tile t
     int v[7] = {0, 0, 0, 0, 0, 0, 0};
+    // unit: tiles per entry of the counts read
+    auto sum = [&](const int2* __restrict__ cnt, const int* at, int unit) {
 #pragma unroll
-    for (int g = 0; g < 3; ++g) {
-        const int nt = (n[g] + kScanTile - 1) / kScanTile;
-        for (int q = (int)threadIdx.x; q < nt; q += kScanThreads) {
-            const int2 w = d.tile_cnt[first[g] + q];
-            v[g] += w.x;
-            if (g != 1) v[g == 0 ? 3 : 4] += w.y;
-            if (g == seg && q < t) {
-                v[5] += w.x;
-                v[6] += w.y;
+        for (int g = 0; g < 3; ++g) {
+            const int nt = (n[g] + kScanTile * unit - 1) / (kScanTile * unit);
+            for (int q = (int)threadIdx.x; q < nt; q += kScanThreads) {
+                const int2 w = cnt[at[g] + q];
+                v[g] += w.x;
+                if (g != 1) v[g == 0 ? 3 : 4] += w.y;
+                if (g == seg && q < t / unit) {
+                    v[5] += w.x;
+                    v[6] += w.y;
+                }
             }
         }
+    };
+    if (sh.tile_groups) {
+        const int gl = tile_groups_of(sh.scan_tiles_l), gh = tile_groups_of(sh.scan_tiles_h);
+        const int at[3] = {0, gl, gl + gh};
+        sum(d.tile_sum, at, kTileGroup);
+        // the tiles before t in its own group
+        const int q = (t & ~(kTileGroup - 1)) + (int)threadIdx.x;
+        if (q < t) {
+            const int2 w = d.tile_cnt[first[seg] + q];
+            v[5] += w.x;
+            v[6] += w.y;
+        }
+    } else {
+        sum(d.tile_cnt, first, 1);
     }
     for (int off = 32; off > 0; off >>= 1) {
 #pragma unroll
@@ -2630,6 +2680,8 @@ void launch_step(const DevState& base, const StepShape& sh, void* stream,
     // the cap can bind only where cap_high < 4 cap_low: a scene's groups
     // and candidates never exceed its low ids
     if (sh.cap_binds) k_cap<<<sh.S, 256, 0, st>>>(d);
+    if (sh.tile_groups && !sh.copy_only)
+        k_tile_sums<<<sh.tile_groups, kScanThreads, 0, st>>>(d, sh);
     const int ntiles = sh.scan_tiles_l + sh.scan_tiles_h + sh.scan_tiles_g;
     auto end = [&](int nfin, int tiles) {
         k_end_step<<<nfin + tiles, kScanThreads, 0, st>>>(d, sh, nfin, vals, d.list_g[par],
