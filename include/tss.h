@@ -272,9 +272,20 @@ typedef struct tss_tuning {
 int tss_set_grid_sort(tss_solver* s, int path);
 int tss_batch_set_grid_sort(tss_batch* b, int path);
 /* Launch shapes and autotuner of a single-scene solver (as for batches,
- * tss_batch_autotune below). */
+ * tss_batch_autotune below).
+ * The shapes are those of neighbour sums with one lane per target. A small
+ * batch takes several (tss_get_lanes: 8, 4 or 1), for which one per target
+ * leaves the chip idle, and none of the shapes: there tss_get_tuning and the
+ * autotuner's result name shapes that no launch uses. Setting shapes
+ * (tss_set_tuning, whichever, also those in force) makes the batch take one
+ * lane per target from then on; the autotuner's pick does not.
+ * tss_reset_tuning brings back the default shapes and the choice of lanes. A
+ * program that keeps shapes for later runs applies them where tss_get_lanes
+ * gives 1. Results depend on none of this. */
 int tss_get_tuning(tss_solver* s, tss_tuning* out);
 int tss_set_tuning(tss_solver* s, const tss_tuning* t);
+int tss_reset_tuning(tss_solver* s);
+int tss_get_lanes(tss_solver* s, int* lanes);
 int tss_autotune(tss_solver* s, int steps_per_trial, int rounds,
                  tss_tuning* out, int* steps_taken, float* trial_log,
                  int log_rows, int* n_log);
@@ -314,6 +325,8 @@ int tss_batch_synchronize(tss_batch* b);
 int tss_batch_num_scenes(tss_batch* b, int* n);
 int tss_batch_get_tuning(tss_batch* b, tss_tuning* out);
 int tss_batch_set_tuning(tss_batch* b, const tss_tuning* t);
+int tss_batch_reset_tuning(tss_batch* b);
+int tss_batch_get_lanes(tss_batch* b, int* lanes);
 /* Autotuner: times candidate shapes with hipEvents while advancing the
  * batch by real steps (they count, the results being shape-independent).
  * After one ordinary step, stage 1 tries every block x depth under the XCD

@@ -199,6 +199,8 @@ PROTOTYPES = {
     "tss_batch_set_grid_sort": (_I, [_P, _I]),
     "tss_get_tuning": (_I, [_P, C.POINTER(TssTuning)]),
     "tss_set_tuning": (_I, [_P, C.POINTER(TssTuning)]),
+    "tss_reset_tuning": (_I, [_P]),
+    "tss_get_lanes": (_I, [_P, C.POINTER(_I)]),
     "tss_autotune": (_I, [_P, _I, _I, C.POINTER(TssTuning), C.POINTER(_I), _P,
                           _I, C.POINTER(_I)]),
     "tss_destroy": (None, [_P]),
@@ -229,6 +231,8 @@ PROTOTYPES = {
     "tss_batch_num_scenes": (_I, [_P, C.POINTER(_I)]),
     "tss_batch_get_tuning": (_I, [_P, C.POINTER(TssTuning)]),
     "tss_batch_set_tuning": (_I, [_P, C.POINTER(TssTuning)]),
+    "tss_batch_reset_tuning": (_I, [_P]),
+    "tss_batch_get_lanes": (_I, [_P, C.POINTER(_I)]),
     "tss_batch_autotune": (_I, [_P, _I, _I, C.POINTER(TssTuning),
                                 C.POINTER(_I), _P, _I, C.POINTER(_I)]),
     "tss_batch_destroy": (None, [_P]),

@@ -225,8 +225,9 @@ struct tss_batch {
     std::vector<SceneHost> scenes;
     RangeAlloc a_low, a_bnd, a_cl, a_ch;
     hipGraphExec_t graph[2] = {nullptr, nullptr};
-    tss::PairTune tune[tss::kPairKernels] = {
-        {256, 16, 0, 0}, {256, 16, 0, 0}, {256, 16, 0, 0}, {256, 16, 0, 0}};
+    static constexpr tss::PairTune kDefaultTune = {256, 16, 0, 0};
+    tss::PairTune tune[tss::kPairKernels] = {kDefaultTune, kDefaultTune, kDefaultTune,
+                                             kDefaultTune};
     bool shapes_set = false;        // launch shapes set by the caller
     bool raw_ptr = false;           // a device pointer was handed out
     bool high_seen = false;         // high particles or groups came from the host
@@ -1050,6 +1051,13 @@ struct tss_batch {
         for (int k = 0; k < tss::kPairKernels; ++k) validate_tune(t[k]);
         for (int k = 0; k < tss::kPairKernels; ++k) tune[k] = t[k];
         shapes_set = true;
+        update_shape();
+    }
+
+    // the default shapes, and the batch's own choice of lanes per target
+    void reset_tuning() {
+        for (tss::PairTune& t : tune) t = kDefaultTune;
+        shapes_set = false;
         update_shape();
     }
 
@@ -2376,6 +2384,20 @@ int tss_batch_set_tuning(tss_batch* b, const tss_tuning* t) {
     });
 }
 
+int tss_batch_reset_tuning(tss_batch* b) {
+    return guarded([&] {
+        require(b, "null argument");
+        b->reset_tuning();
+    });
+}
+
+int tss_batch_get_lanes(tss_batch* b, int* lanes) {
+    return guarded([&] {
+        require(b && lanes, "null argument");
+        *lanes = b->sh.coop ? b->sh.coop : 1;
+    });
+}
+
 int tss_batch_autotune(tss_batch* b, int steps_per_trial, int rounds, tss_tuning* out,
                        int* steps_taken, float* trial_log, int log_rows, int* n_log) {
     return guarded([&] {
@@ -2418,6 +2440,12 @@ int tss_set_tuning(tss_solver* s, const tss_tuning* t) {
         tune_from_abi(t, pt);
         s->b.set_tuning(pt);
     });
+}
+
+int tss_reset_tuning(tss_solver* s) { return tss_batch_reset_tuning(s ? &s->b : nullptr); }
+
+int tss_get_lanes(tss_solver* s, int* lanes) {
+    return tss_batch_get_lanes(s ? &s->b : nullptr, lanes);
 }
 
 int tss_autotune(tss_solver* s, int steps_per_trial, int rounds, tss_tuning* out,

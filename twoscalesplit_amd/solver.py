@@ -239,7 +239,18 @@ class Solver:
         return t
 
     def set_tuning(self, t: N.TssTuning) -> None:
+        """Launch shapes; one lane per target from then on (tss_set_tuning)."""
         N.check(N.lib().tss_set_tuning(self._h, C.byref(t)), "set_tuning")
+
+    def reset_tuning(self) -> None:
+        """Default shapes and the solver's own choice of lanes per target."""
+        N.check(N.lib().tss_reset_tuning(self._h), "reset_tuning")
+
+    def lanes(self) -> int:
+        """Lanes per target of a step's neighbour sums: 8, 4 or 1."""
+        n = C.c_int()
+        N.check(N.lib().tss_get_lanes(self._h, C.byref(n)), "lanes")
+        return n.value
 
     def set_grid_sort(self, path: int) -> None:
         """Sort of the grid build: N.SORT_AUTO, SORT_RADIX, SORT_COUNT or
@@ -418,8 +429,20 @@ class Batch:
         N.check(N.lib().tss_batch_set_grid_sort(self._h, path), "set_grid_sort")
 
     def set_tuning(self, t: N.TssTuning) -> None:
+        """Launch shapes; one lane per target from then on."""
         N.check(N.lib().tss_batch_set_tuning(self._h, C.byref(t)),
                 "tss_batch_set_tuning")
+
+    def reset_tuning(self) -> None:
+        """Default shapes and the batch's own choice of lanes per target."""
+        N.check(N.lib().tss_batch_reset_tuning(self._h), "tss_batch_reset_tuning")
+
+    def lanes(self) -> int:
+        """Lanes per target of a step's neighbour sums: 8, 4 or 1."""
+        n = C.c_int()
+        N.check(N.lib().tss_batch_get_lanes(self._h, C.byref(n)),
+                "tss_batch_get_lanes")
+        return n.value
 
     def autotune(self, steps_per_trial: int = 1, rounds: int = 2) -> dict:
         """Native autotuner (advances every scene by real steps)."""
