@@ -9,7 +9,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from twoscalesplit_amd import MODE_BAND, Batch, Solver, _native as N, scenes
+from twoscalesplit_amd import MODE_BAND, MODE_PLAIN, MODE_REFERENCE, Batch, Solver, _native as N, scenes
 
 FIELDS = ("POS_L", "VEL_L", "RHO_L", "POS_H", "RHO_H", "LIST_L", "LIST_H", "LIST_G")
 
@@ -70,3 +70,20 @@ def test_batch():
         assert b.counts(one)["step"] == 3
     finally:
         b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode,split_x,last", [
+    (MODE_PLAIN, 0.0, (16384, 49152)), (MODE_BAND, -1.0, (16384, 49152)),
+    (MODE_REFERENCE, 0.1, (5461, 16384)),
+    # all split: the plane lies before the domain or on its edge
+    (MODE_REFERENCE, 0.0, (5461, 12288)), (MODE_REFERENCE, -1.0, (5461, 12288))])
+def test_lines(mode, split_x, last):
+    """The capacities up to which a scene takes eight and four lanes."""
+    sc = scenes.small_two_scale(nx=4, ny=4, mode=mode, split_x=split_x)
+    got = []
+    for cap in (last[0], last[0] + 1, last[1], last[1] + 1):
+        sol = Solver(sc.cfg, sc.low_xy, cap, sc.bnd_xy)
+        got.append(sol.lanes())
+        sol.close()
+    assert got == [8, 4, 4, 1]

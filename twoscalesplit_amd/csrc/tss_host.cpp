@@ -538,16 +538,24 @@ struct tss_batch {
         // (and three at once, on their streams): plain 8k 82/-/54
         // (30/-/21), 16k 83/-/57 (30/-/23), 32k 84/66/- (32/28/-), 48k
         // 84/72/- (34/34/-), 64k 86/104/- (35/51/-); half split 4k 94/-/62
-        // (34/-/24), 8k 98/71/68 (36/29/30), 16k 96/78/- (38/37/-), 20k
-        // 98/89/- (40/46/-), 24k 105/95/- (43/51/-); all split 4k 83/-/61
-        // (30/-/24), 8k 85/73/74 (33/31/35), 12k 87/82/- (35/39/-), 16k 91/93/- (37/48/-), 20k
-        // 93/105/- (39/58/-)
-        long long expect = 0;
-        for (const SceneHost& s : scenes)
-            if (s.alive) expect += (s.cfg.mode == TSS_MODE_REFERENCE ? 3LL : 1LL) * s.lcap;
-        sh.coop = shapes_set || expect > tss::kCoop4Targets ? 0
-                  : expect > tss::kCoop8Targets             ? 4
-                                                            : 8;
+        // (34/-/24), 8k 98/71/68 (36/29/30), 16k 96/78/- (37/37/-), 20k
+        // 98/89/- (40/46/-); three quarters split 14k 102/84/- (40/39/-),
+        // 16k 101/90/- (39/45/-). All split, 4k 84/67/61 (30/26/24), 5.4k
+        // 84/69/67 (31/27/29), 9.5k 86/73/- (34/34/-), 12k 88/81/- (35/39/-),
+        // 14k 89/87/- (36/43/-), 16k 90/92/- (37/49/-): three at once lose
+        // from 9.5k on and one alone from 14k, so there an id counts as four
+        // against the upper line
+        long long expect8 = 0, expect4 = 0;
+        for (const SceneHost& s : scenes) {
+            if (!s.alive) continue;
+            const bool two = s.cfg.mode == TSS_MODE_REFERENCE;
+            const bool all = two && s.cfg.split_x <= s.cfg.domain_origin[0];
+            expect8 += (two ? 3LL : 1LL) * s.lcap;
+            expect4 += (all ? 4LL : two ? 3LL : 1LL) * s.lcap;
+        }
+        sh.coop = shapes_set || expect4 > tss::kCoop4Targets ? 0
+                  : expect8 > tss::kCoop8Targets             ? 4
+                                                             : 8;
         sh.relax_iters = 0;
         for (auto& s : scenes)
             if (s.alive) sh.relax_iters = std::max(sh.relax_iters, s.cfg.relax_iters);
