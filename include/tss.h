@@ -335,9 +335,12 @@ int tss_batch_get_lanes(tss_batch* b, int* lanes);
  * `rounds` times for
  * steps_per_trial steps, in alternating order; a candidate's time per
  * target of the kernel's level is its fastest trial, and per kernel the
- * fastest candidate is kept (and returned in out).
+ * fastest candidate is kept (and returned in out). Levels that share a launch
+ * in a step (tss_tuning) share it in the trials, and its time per target of
+ * both picks one shape for both.
  * steps_taken: steps advanced. trial_log (optional): log_rows x 8 floats per
- * trial, (block, depth, xcd_order, grid, ms of kernels 0..3); n_log rows. */
+ * trial, (block, depth, xcd_order, grid, ms of kernels 0..3; a shared
+ * launch's ms at both of its levels); n_log rows. */
 int tss_batch_autotune(tss_batch* b, int steps_per_trial, int rounds,
                        tss_tuning* out, int* steps_taken, float* trial_log,
                        int log_rows, int* n_log);

@@ -271,6 +271,7 @@ struct StepShape {
     int tile_groups;          // groups of them summed first, 0: none (tile_totals)
     PairTune tune[kPairKernels];
     int coop;                 // neighbour sums: 8 or 4 lanes per target, 0: one (PairTune)
+    int trial;                // 1: timed steps share the levels' launches like untimed ones
     int S;
     int red_slots;            // chunk slots in use (grid of the reduction)
     int list_parity;          // which list buffer holds the current lists
@@ -304,6 +305,15 @@ constexpr int kWorkCounts = 13;
 // Kernel launchers (tss_kernels.hip). All enqueue on `stream`.
 // timing_events: hipEvent_t[kTimingPoints] or nullptr; event_flags is passed
 // to hipEventRecordWithFlags (hipEventRecordExternal under graph capture).
+// Whether a step without timing points runs both levels of the force (density)
+// in one launch, given equal block and depth (kBothLevelsCap).
+inline bool shares_force(const StepShape& sh) {
+    return !sh.coop && sh.two && sh.cap_alive <= kBothLevelsCap;
+}
+inline bool shares_density(const StepShape& sh) {
+    return shares_force(sh) || (!sh.coop && sh.band_any);
+}
+
 void launch_step(const DevState& d, const StepShape& sh, void* stream,
                  void* timing_events, unsigned int event_flags);
 void launch_neighbors_n(const DevState& d, const StepShape& sh, int scene,

@@ -1076,7 +1076,12 @@ struct tss_batch {
     // step, candidates are visited `rounds` times in alternating order; the
     // lowest mean time per target wins, per kernel. Stage 1: block x depth
     // with the plain grid; stage 2: XCD block order x persistent grid caps on
-    // top of each kernel's stage-1 winner.
+    // top of each kernel's stage-1 winner. Levels that share a launch in an
+    // untimed step share it in the trials: its time per target of both levels
+    // decides for both, so the pick keeps them together (picked one by one,
+    // blocks and depths usually differ and the launches part: us per step
+    // untuned / picked one by one / together, half split 32k 104/99 to 126/98,
+    // 100k 151/155 to 170/143, all split 20k 92/132/87, 100k 164/196/161).
     int autotune(int steps, int rounds, float* trial_log, int log_cap, int* n_log) {
         require(steps >= 1 && rounds >= 1, "autotune: steps and rounds must be >= 1");
         int alive = 0;
@@ -1090,6 +1095,10 @@ struct tss_batch {
         HIP_CHECK(hipGetDevice(&dev));
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         int taken = 0, logged = 0;
+        struct Trials {  // ends the trials' launches, by an exception too
+            int& on;
+            ~Trials() { on = 0; }
+        } trials{sh.trial};
         // per-target time of each kernel: the population changes from step to
         // step (the first step of a scene splits before any child exists),
         // so a trial's kernel time is divided by the targets of its level in
@@ -1105,13 +1114,20 @@ struct tss_batch {
                     const size_t c = (r & 1) ? cand.size() - 1 - i : i;
                     set_tuning(cand[c].data());
                     set_timing(true);
+                    sh.trial = 1;
                     step_eager(steps);
                     taken += steps;
                     float ph[kPhases];
                     phase_times(ph);
                     const tss::DevCounts dc = read_counts();
-                    const int ntg[tss::kPairKernels] = {dc.n_l_last, dc.n_h_last, dc.n_l_last,
-                                                        dc.n_h_last};
+                    int ntg[tss::kPairKernels] = {dc.n_l_last, dc.n_h_last, dc.n_l_last,
+                                                  dc.n_h_last};
+                    auto shared = [&](int low) {
+                        ph[1 + low] = ph[2 + low] = ph[1 + low] + ph[2 + low];
+                        ntg[low] = ntg[low + 1] = ntg[low] + ntg[low + 1];
+                    };
+                    if (tss::shares_density(sh)) shared(tss::kTuneDensityLow);
+                    if (tss::shares_force(sh)) shared(tss::kTuneForceLow);
                     for (int k = 0; k < tss::kPairKernels; ++k) {
                         if (ntg[k] <= 0) continue;
                         tot[c][k] = std::min(tot[c][k], (double)ph[1 + k] / (double)ntg[k]);

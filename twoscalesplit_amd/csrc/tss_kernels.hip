@@ -2633,25 +2633,28 @@ void launch_step(const DevState& base, const StepShape& sh, void* stream,
     else if (sh.coop == 4)
         launch_coop<4>(d, sh, vals, keys, st, ev == nullptr, mark);
     else {
-        const bool force_both = sh.two && !ev && sh.cap_alive <= kBothLevelsCap;
-        const bool density_both = force_both || (sh.band_any && !ev);
-        if (!density_both || !launch_both<false>(d, vals, keys, sh.tune[kTuneDensityLow],
-                                         sh.tune[kTuneDensityHigh], sh.cap_alive, sh.band_any, st)) {
+        const bool share = !ev || sh.trial;
+        const bool density_both =
+            share && shares_density(sh) &&
+            launch_both<false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.tune[kTuneDensityHigh],
+                               sh.cap_alive, sh.band_any, st);
+        if (!density_both)
             launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
-            mark(2);
-            if (sh.two)
-                launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh],
-                                         4 * sh.cap_alive, st, sh.band_any);
-        }
+        mark(2);
+        if (!density_both && sh.two)
+            launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh], 4 * sh.cap_alive,
+                                     st, sh.band_any);
         mark(3);
-        if (!force_both || !launch_both<true>(d, vals, keys, sh.tune[kTuneForceLow],
-                                        sh.tune[kTuneForceHigh], sh.cap_alive, sh.band_any, st)) {
+        const bool force_both =
+            share && shares_force(sh) &&
+            launch_both<true>(d, vals, keys, sh.tune[kTuneForceLow], sh.tune[kTuneForceHigh],
+                              sh.cap_alive, sh.band_any, st);
+        if (!force_both)
             launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
-            mark(4);
-            if (sh.two)
-                launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive,
-                                        st, sh.band_any);
-        }
+        mark(4);
+        if (!force_both && sh.two)
+            launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive, st,
+                                    sh.band_any);
     }
     mark(5);
     // the reductions, split candidates and groups in one launch (two where
