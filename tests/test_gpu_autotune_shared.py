@@ -44,3 +44,26 @@ def test_shared_levels_get_one_shape(mode, cap, density, force):
     finally:
         a.close()
         b.close()
+
+
+def test_refused_autotune_changes_nothing():
+    """A state that host writes left invalid stops the autotuner's first step:
+    timing, shapes and lanes stay as they were."""
+    sc = scenes.small_two_scale(nx=24, ny=30, mode=MODE_BAND)
+    sol = Solver(sc.cfg, sc.low_xy, 720, sc.bnd_xy)
+    try:
+        sol.step(1)
+        lanes, shapes = sol.lanes(), sol.get_tuning().as_dict()
+        sol.enable_timing(True)
+        state = sol.read("STATE_L")
+        bad = state.copy()
+        bad[sol.read("LIST_L")[:1]] = 2
+        sol.write("STATE_L", bad)
+        with pytest.raises(RuntimeError, match="deleted particle listed"):
+            sol.autotune(1, 1)
+        assert sol.lanes() == lanes and sol.get_tuning().as_dict() == shapes
+        sol.write("STATE_L", state)
+        sol.step(2)
+        assert all(v > 0 for v in sol.phase_times().values())
+    finally:
+        sol.close()

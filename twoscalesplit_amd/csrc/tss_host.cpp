@@ -1095,10 +1095,25 @@ struct tss_batch {
         HIP_CHECK(hipGetDevice(&dev));
         HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         int taken = 0, logged = 0;
-        struct Trials {  // ends the trials' launches, by an exception too
-            int& on;
-            ~Trials() { on = 0; }
-        } trials{sh.trial};
+        // ends the trials; after an exception with the shapes, the choice of
+        // lanes and the timing from before
+        struct Trials {
+            tss_batch& b;
+            bool timing, set, done = false;
+            std::array<tss::PairTune, tss::kPairKernels> shapes;
+            ~Trials() {
+                b.sh.trial = 0;
+                if (done) return;
+                std::copy(shapes.begin(), shapes.end(), b.tune);
+                b.shapes_set = set;
+                try {
+                    b.update_shape();
+                    b.set_timing(timing);
+                } catch (...) {  // a device error: the first one is reported
+                }
+            }
+        } trials{*this, was_timing, were_set};
+        std::copy(tune, tune + tss::kPairKernels, trials.shapes.begin());
         // per-target time of each kernel: the population changes from step to
         // step (the first step of a scene splits before any child exists),
         // so a trial's kernel time is divided by the targets of its level in
@@ -1190,6 +1205,7 @@ struct tss_batch {
         shapes_set = were_set;
         update_shape();
         set_timing(was_timing);
+        trials.done = true;
         if (n_log) *n_log = logged;
         return taken;
     }
