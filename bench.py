@@ -413,7 +413,8 @@ def main() -> int:
     n0 = c0["n_low"] + c0["n_high"]
 
     # timed region: K graph-replayed steps; hipEvents inside the graphs
-    # time every phase of every step on the solver's stream
+    # time every phase of every step on the solver's stream (a timed step has
+    # a launch per phase, where an untimed one merges some)
     sol.enable_timing(True)
     _log("timed", args.steps, "steps of", n0, "particles")
     t0 = time.perf_counter()

@@ -224,8 +224,12 @@ int tss_pair_sets(tss_solver* s, int level, uint32_t* counts, uint32_t* sums,
  * relaxation of new children when a scene enables it) [1] density, low
  * targets [2] density, high targets [3] force + integration, low targets
  * [4] force + integration, high targets [5] FP64 reductions [6] adaptivity
- * and list compaction [7] finalize (counts, dt). tss_enable_timing resets
- * the averages. No counterpart in the reference (it times nothing). */
+ * and list compaction [7] finalize (counts, dt). A timed step has a launch per
+ * phase; an untimed one runs [5] with the adaptivity of [6], the compaction
+ * with [7], and on many batches both levels of [1], [2] and of [3], [4] (see
+ * tss_tuning and tss_get_lanes) in one launch each, so it takes less than the
+ * sum of the phases. tss_enable_timing resets the averages. No counterpart in
+ * the reference (it times nothing). */
 #define TSS_PHASE_COUNT 8
 int tss_enable_timing(tss_solver* s, int on);
 int tss_phase_times(tss_solver* s, float out_ms[TSS_PHASE_COUNT]);
@@ -244,11 +248,13 @@ int tss_work_counts(tss_solver* s, unsigned long long out[TSS_WORK_COUNT]);
  * or 512 threads; depth: LDS buffer depth, 8, 16 or 32 pairs per lane;
  * xcd_order: 1 gives each of the 8 XCDs one contiguous range of blocks;
  * grid: 0 = one thread per target of capacity (high targets of a batch with a
- * band-rule scene: of 262144 at most), else a persistent grid of at
- * most this many blocks. Equal block and depth of both levels let them share
- * a launch on batches of up to 262144 low ids. Results never depend on the shapes (every
- * neighbour sum is lane-local). Default: 256, 16, 0, 0. No counterpart in
- * the reference (fixed 256-thread blocks, R/WCSPHSolver.cu:2421). */
+ * band-rule scene: of 262144 at most), else a persistent grid of at most this
+ * many blocks. Equal block and depth of both levels let them share a launch:
+ * density and force of two-level batches of up to 262144 low ids, the density
+ * of batches with a band-rule scene of any size. Results never depend on the
+ * shapes (every neighbour sum is lane-local). Default: 256, 16, 0, 0. No
+ * counterpart in the reference (fixed 256-thread blocks,
+ * R/WCSPHSolver.cu:2421). */
 typedef struct tss_tuning {
     int block[4];
     int depth[4];
