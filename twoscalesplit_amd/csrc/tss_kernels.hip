@@ -1736,38 +1736,36 @@ __device__ __forceinline__ TileTotals tile_totals(const DevState& d, const StepS
                                                   int t, int (*lds)[8]) {
     const DevCounts* c = d.counts;
     const int n[3] = {c->n_l, c->n_h, c->n_g};
-    const int first[3] = {0, sh.scan_tiles_l, sh.scan_tiles_l + sh.scan_tiles_h};
+    // counts of groups of tiles where those were summed, else of tiles
+    const bool groups = sh.tile_groups != 0;
+    const int2* __restrict__ cnt = groups ? d.tile_sum : d.tile_cnt;
+    const int ul = groups ? tile_groups_of(sh.scan_tiles_l) : sh.scan_tiles_l;
+    const int uh = groups ? tile_groups_of(sh.scan_tiles_h) : sh.scan_tiles_h;
+    const int first[3] = {0, ul, ul + uh};
+    const int tu = groups ? t / kTileGroup : t;
     // entries not kept, P1 (high tiles have none), and both before tile t
     int v[7] = {0, 0, 0, 0, 0, 0, 0};
-    // unit: tiles per entry of the counts read
-    auto sum = [&](const int2* __restrict__ cnt, const int* at, int unit) {
 #pragma unroll
-        for (int g = 0; g < 3; ++g) {
-            const int nt = (n[g] + kScanTile * unit - 1) / (kScanTile * unit);
-            for (int q = (int)threadIdx.x; q < nt; q += kScanThreads) {
-                const int2 w = cnt[at[g] + q];
-                v[g] += w.x;
-                if (g != 1) v[g == 0 ? 3 : 4] += w.y;
-                if (g == seg && q < t / unit) {
-                    v[5] += w.x;
-                    v[6] += w.y;
-                }
+    for (int g = 0; g < 3; ++g) {
+        const int tiles = (n[g] + kScanTile - 1) / kScanTile;
+        const int nt = groups ? tile_groups_of(tiles) : tiles;
+        for (int q = (int)threadIdx.x; q < nt; q += kScanThreads) {
+            const int2 w = cnt[first[g] + q];
+            v[g] += w.x;
+            if (g != 1) v[g == 0 ? 3 : 4] += w.y;
+            if (g == seg && q < tu) {
+                v[5] += w.x;
+                v[6] += w.y;
             }
         }
-    };
-    if (sh.tile_groups) {
-        const int gl = tile_groups_of(sh.scan_tiles_l), gh = tile_groups_of(sh.scan_tiles_h);
-        const int at[3] = {0, gl, gl + gh};
-        sum(d.tile_sum, at, kTileGroup);
-        // the tiles before t in its own group
-        const int q = (t & ~(kTileGroup - 1)) + (int)threadIdx.x;
-        if (q < t) {
-            const int2 w = d.tile_cnt[first[seg] + q];
-            v[5] += w.x;
-            v[6] += w.y;
-        }
-    } else {
-        sum(d.tile_cnt, first, 1);
+    }
+    // and the tiles before t in its own group
+    const int q = (t & ~(kTileGroup - 1)) + (int)threadIdx.x;
+    if (groups && q < t) {
+        const int2 w = d.tile_cnt[(seg == 0 ? 0 : seg == 1 ? sh.scan_tiles_l
+                                                 : sh.scan_tiles_l + sh.scan_tiles_h) + q];
+        v[5] += w.x;
+        v[6] += w.y;
     }
     for (int off = 32; off > 0; off >>= 1) {
 #pragma unroll
