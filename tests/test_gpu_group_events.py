@@ -11,6 +11,8 @@ import time
 import numpy as np
 import pytest
 
+from parity import check_step
+
 from twoscalesplit_amd import MODE_BAND, MODE_REFERENCE, Batch, Solver, scenes
 
 pytestmark = pytest.mark.gpu
@@ -133,3 +135,56 @@ def test_splitting_all_costs_little():
         us[split_x] = best * 1e6
     print("[us]", us, flush=True)
     assert us[-1.0] < us[100.0] + 320.0
+
+
+@pytest.mark.parametrize("ny,many", [(160, False), (163, False), (164, True),
+                                     (180, True)])
+def test_more_groups_than_a_wave_per_block(ny, many):
+    """A band as wide as the scene: up to 32768 groups a block of their launch
+    takes one wave of them, beyond that whole blocks; steps as the oracle's."""
+    sc = scenes.small_two_scale(nx=200, ny=ny, nxd=440, nyd=ny + 40, mode=MODE_BAND)
+    h = sc.cfg.effective_radius
+    sc.cfg.band_radius, sc.cfg.merge_radius = 60 * h, 12 * h
+    sc.cfg.promote_min_age, sc.cfg.promote_max_age = 2, 3
+    print("[case]", ny, flush=True)
+    sol = Solver(sc.cfg, sc.low_xy, len(sc.low_xy), sc.bnd_xy)
+    seen = dict.fromkeys(COUNTS, 0)
+    try:
+        sol.step(1)
+        assert (sol.counts()["n_groups"] > 32768) == many
+        for _ in range(4):
+            check_step(sol, sc.cfg, sc.bnd_xy, pairs=False)
+            for k in COUNTS:
+                seen[k] += sol.counts()[k]
+    finally:
+        sol.close()
+    print("[seen]", seen, flush=True)
+    assert seen["n_dissolve"] > 0 and seen["n_promote"] > 0
+
+
+def test_many_groups_cost():
+    """300,000 groups, whose band tests are long, took 3.6 ms a step in blocks of
+    one wave beside the reductions, 2.4 ms in whole blocks: 3.2 and 2.1 ms
+    more than a step of the same scene with few."""
+    us = {}
+    for wide in (False, True):
+        sc = scenes.c3_large(forced=False)
+        sc.cfg.dt_mode, sc.cfg.time_step = 0, 1e-6
+        if wide:
+            h = sc.cfg.effective_radius
+            sc.cfg.band_radius, sc.cfg.merge_radius = 40 * h, 41 * h
+        sol = Solver(sc.cfg, sc.low_xy, sc.cap_low, sc.bnd_xy)
+        try:
+            sol.step(4)
+            us[wide] = np.inf
+            for _ in range(6):
+                sol.synchronize()
+                t = time.perf_counter()
+                sol.step(1)
+                sol.synchronize()
+                us[wide] = min(us[wide], (time.perf_counter() - t) * 1e6)
+            assert (sol.counts()["n_groups"] > 200000) == wide
+        finally:
+            sol.close()
+    print("[us]", us, flush=True)
+    assert us[True] < us[False] + 2600.0

@@ -1587,6 +1587,13 @@ __device__ __forceinline__ void update_groups(const DevState& d, const uint32_t*
     }
 }
 
+// Groups up to which a block of k_adapt takes one wave of them under the band
+// rule: 2048 waves, which is what eight blocks on each of 256 CUs hold. us of
+// adaptivity and compaction, one wave / whole blocks: 20k groups 70/75, 25k
+// 138/145, 41k 99/90, 55k 203/152, 128k 485/366, 301k 2583/1826 (in a launch
+// of their own, blocks of one wave, 2015).
+constexpr int kSpreadGroups = 32768;
+
 // What follows the force pass and does not depend on each other, in one
 // launch: blocks [0, nred) the reductions, the next nsplit the split
 // candidates, the others the groups. (Three launches took 8 + 4.5 + 4.5 us on
@@ -1602,13 +1609,14 @@ __global__ __launch_bounds__(256) void k_adapt(DevState d, const uint32_t* __res
     } else if (b < nred + nsplit) {
         split_candidates(d, b - nred, nsplit);
     } else {
-        // few groups and long band tests: a lane per child, and one wave per
-        // block to spread them over the CUs
-        constexpr int kUse = LANES == 4 ? 64 : 256;
-        if ((int)threadIdx.x < kUse)
+        // long band tests: a lane per child, and one wave per block to spread
+        // few groups over the CUs; more than kSpreadGroups fill the resident
+        // blocks (eight per CU, by the reductions' LDS) with whole ones
+        const int use = LANES == 4 && d.counts->n_g <= kSpreadGroups ? 64 : 256;
+        if ((int)threadIdx.x < use)
             update_groups<LANES>(d, vals, list_g, solo, th, tg,
-                                 (b - nred - nsplit) * kUse + (int)threadIdx.x,
-                                 ((int)gridDim.x - nred - nsplit) * kUse);
+                                 (b - nred - nsplit) * use + (int)threadIdx.x,
+                                 ((int)gridDim.x - nred - nsplit) * use);
     }
 }
 
