@@ -248,10 +248,11 @@ int tss_work_counts(tss_solver* s, unsigned long long out[TSS_WORK_COUNT]);
  * or 512 threads; depth: LDS buffer depth, 8, 16 or 32 pairs per lane;
  * xcd_order: 1 gives each of the 8 XCDs one contiguous range of blocks;
  * grid: 0 = one thread per target of capacity (high targets of a batch with a
- * band-rule scene: of 262144 at most), else a persistent grid of at most this
- * many blocks. Equal block and depth of both levels let them share a launch:
- * density and force of two-level batches of up to 262144 low ids, the density
- * of batches with a band-rule scene of any size. Results never depend on the
+ * band-rule scene and at most 65536 low ids of the reference rule: of 262144
+ * at most), else a persistent grid of at most this many blocks. Equal block
+ * and depth of both levels let them share a launch: density and force of
+ * two-level batches of up to 262144 low ids, and the density of such batches
+ * with a band-rule scene of any size. Results never depend on the
  * shapes (every neighbour sum is lane-local). Default: 256, 16, 0, 0. No
  * counterpart in the reference (fixed 256-thread blocks,
  * R/WCSPHSolver.cu:2421). */

@@ -253,8 +253,18 @@ constexpr long long kCoop4Targets = 49152;
 // the low ones): 400k 156/154 (102/101), 1M 294/292 (243/241), 64 scenes of
 // 2k to 64k with 50k high particles 507/485 (351/347); the force as above
 // (both shared: 1M 293 (243), and 505 us for two steps of it on launch shapes
-// set for large scenes against 492).
+// set for large scenes against 492); not where sparse_high says otherwise.
 constexpr long long kBothLevelsCap = 262144;
+
+// Under the band rule the high level is sparse (some ten thousand targets in a
+// grid of four per low id): its blocks are cut to this many targets and loop
+// where there are more, instead of tens of thousands of empty blocks waiting
+// for LDS (band rule at 400k, us per step alone and three at once: 159 -> 156
+// and 104 -> 102, at 1M 301 -> 294 and 249 -> 243). Not beside scenes of the
+// reference rule that may list more than these (sparse_high): a scene of 1M
+// that all splits with one of 2k under the band rule 1226 us cut and 1136
+// whole, 200k 303 and 283, 100k 191 and 172 (untuned 172 and 175).
+constexpr long long kSparseTargets = 262144;
 
 // Host-known launch parameters of one step.
 struct StepShape {
@@ -279,6 +289,8 @@ struct StepShape {
     int clear_blocks;         // blocks of the cell-table clear (clear_blk)
     int cap_binds;            // 1: a resident scene has cap_high < 4 cap_low
     int band_any;             // 1: a resident scene uses the surface band rule
+    int sparse_high;          // 1: and reference-rule scenes list at most
+                              // kSparseTargets high targets
     int two;                  // 1: high particles or groups may be listed
     int copy_only;            // 1: no entry can leave or join a list (not two,
                               // and no raw device pointer handed out)
@@ -311,7 +323,7 @@ inline bool shares_force(const StepShape& sh) {
     return !sh.coop && sh.two && sh.cap_alive <= kBothLevelsCap;
 }
 inline bool shares_density(const StepShape& sh) {
-    return shares_force(sh) || (!sh.coop && sh.band_any);
+    return shares_force(sh) || (!sh.coop && sh.sparse_high);
 }
 
 void launch_step(const DevState& d, const StepShape& sh, void* stream,

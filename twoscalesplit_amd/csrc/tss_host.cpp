@@ -492,10 +492,13 @@ struct tss_batch {
                                    groups(sh.scan_tiles_g);
         sh.cap_binds = 0;
         sh.band_any = 0;
+        long long split_cap = 0;  // low ids of the reference rule
         for (const SceneHost& s : scenes) {
             if (s.alive && effective_cap_high(s.cfg, s.lcap) < 4LL * s.lcap) sh.cap_binds = 1;
-            if (s.alive && s.cfg.mode == 2) sh.band_any = 1;
+            if (s.alive && s.cfg.mode == TSS_MODE_BAND) sh.band_any = 1;
+            if (s.alive && s.cfg.mode == TSS_MODE_REFERENCE) split_cap += s.lcap;
         }
+        sh.sparse_high = sh.band_any && 4 * split_cap <= tss::kSparseTargets;
         long long maxkey = 1;
         for (auto& s : scenes)
             if (s.alive) maxkey = std::max<long long>(maxkey, (long long)s.cbh + s.nch);

@@ -2654,24 +2654,24 @@ void launch_step(const DevState& base, const StepShape& sh, void* stream,
         const bool density_both =
             share && shares_density(sh) &&
             launch_both<false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.tune[kTuneDensityHigh],
-                               sh.cap_alive, sh.band_any, st);
+                               sh.cap_alive, sh.sparse_high, st);
         if (!density_both)
             launch_pair<false, false>(d, vals, keys, sh.tune[kTuneDensityLow], sh.cap_alive, st);
         mark(2);
         if (!density_both && sh.two)
             launch_pair<false, true>(d, vals, keys, sh.tune[kTuneDensityHigh], 4 * sh.cap_alive,
-                                     st, sh.band_any);
+                                     st, sh.sparse_high);
         mark(3);
         const bool force_both =
             share && shares_force(sh) &&
             launch_both<true>(d, vals, keys, sh.tune[kTuneForceLow], sh.tune[kTuneForceHigh],
-                              sh.cap_alive, sh.band_any, st);
+                              sh.cap_alive, sh.sparse_high, st);
         if (!force_both)
             launch_pair<true, false>(d, vals, keys, sh.tune[kTuneForceLow], sh.cap_alive, st);
         mark(4);
         if (!force_both && sh.two)
             launch_pair<true, true>(d, vals, keys, sh.tune[kTuneForceHigh], 4 * sh.cap_alive, st,
-                                    sh.band_any);
+                                    sh.sparse_high);
     }
     mark(5);
     // the reductions, split candidates and groups in one launch (two where
