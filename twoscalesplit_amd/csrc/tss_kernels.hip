@@ -1734,29 +1734,29 @@ __global__ __launch_bounds__(kScanThreads) void k_tile_sums(DevState d, StepShap
 }
 
 // P0 and P1 totals of the segments, and of the tiles of segment `seg` before
-// its tile `t`; the same on every thread. lds: 7 ints per wave.
+// its tile `t`; the same on every thread. lds: 7 ints per wave. GROUPS: from
+// the groups of tiles that k_tile_sums summed.
 struct TileTotals {
     int keep[3], p1[3];  // low, high, group
     int before0, before1;
 };
 
+template <bool GROUPS>
 __device__ __forceinline__ TileTotals tile_totals(const DevState& d, const StepShape& sh, int seg,
                                                   int t, int (*lds)[8]) {
     const DevCounts* c = d.counts;
     const int n[3] = {c->n_l, c->n_h, c->n_g};
-    // counts of groups of tiles where those were summed, else of tiles
-    const bool groups = sh.tile_groups != 0;
-    const int2* __restrict__ cnt = groups ? d.tile_sum : d.tile_cnt;
-    const int ul = groups ? tile_groups_of(sh.scan_tiles_l) : sh.scan_tiles_l;
-    const int uh = groups ? tile_groups_of(sh.scan_tiles_h) : sh.scan_tiles_h;
+    const int2* __restrict__ cnt = GROUPS ? d.tile_sum : d.tile_cnt;
+    const int ul = GROUPS ? tile_groups_of(sh.scan_tiles_l) : sh.scan_tiles_l;
+    const int uh = GROUPS ? tile_groups_of(sh.scan_tiles_h) : sh.scan_tiles_h;
     const int first[3] = {0, ul, ul + uh};
-    const int tu = groups ? t / kTileGroup : t;
+    const int tu = GROUPS ? t / kTileGroup : t;
     // entries not kept, P1 (high tiles have none), and both before tile t
     int v[7] = {0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
     for (int g = 0; g < 3; ++g) {
         const int tiles = (n[g] + kScanTile - 1) / kScanTile;
-        const int nt = groups ? tile_groups_of(tiles) : tiles;
+        const int nt = GROUPS ? tile_groups_of(tiles) : tiles;
         for (int q = (int)threadIdx.x; q < nt; q += kScanThreads) {
             const int2 w = cnt[first[g] + q];
             v[g] += w.x;
@@ -1769,7 +1769,7 @@ __device__ __forceinline__ TileTotals tile_totals(const DevState& d, const StepS
     }
     // and the tiles before t in its own group
     const int q = (t & ~(kTileGroup - 1)) + (int)threadIdx.x;
-    if (groups && q < t) {
+    if (GROUPS && q < t) {
         const int2 w = d.tile_cnt[(seg == 0 ? 0 : seg == 1 ? sh.scan_tiles_l
                                                  : sh.scan_tiles_l + sh.scan_tiles_h) + q];
         v[5] += w.x;
@@ -1804,6 +1804,7 @@ __device__ __forceinline__ TileTotals tile_totals(const DevState& d, const StepS
 }
 
 // One tile of the next lists.
+template <bool GROUPS>
 __device__ __forceinline__ void compact_tile(const DevState& d, const StepShape& sh, int tile,
                                              const uint32_t* __restrict__ vals,
                                              const int* __restrict__ list_g,
@@ -1872,7 +1873,7 @@ __device__ __forceinline__ void compact_tile(const DevState& d, const StepShape&
             wsum[1][q][wv] = __popcll(m1[q]);
         }
     }
-    const TileTotals tt = tile_totals(d, sh, seg, t, lds);  // a barrier inside
+    const TileTotals tt = tile_totals<GROUPS>(d, sh, seg, t, lds);  // a barrier inside
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     const int keepL = tt.keep[0], keepH = tt.keep[1], keepG = tt.keep[2];
     int run0 = tt.before0, run1 = tt.before1;
@@ -1934,6 +1935,7 @@ __device__ __forceinline__ void compact_tile(const DevState& d, const StepShape&
 // the next step's list sizes. The scene's chunk partials are summed in a
 // fixed order (thread t takes slots t, t+256, ...; then a fixed tree), so the
 // sums are bitwise reproducible.
+template <bool GROUPS>
 __device__ __forceinline__ void finalize_scene(const DevState& d, const StepShape& shp, int s,
                                                double (*sh)[256], int (*lds)[8]) {
     SceneDev& sc = d.scenes[s];
@@ -2017,7 +2019,7 @@ __device__ __forceinline__ void finalize_scene(const DevState& d, const StepShap
     if (s == 0) {
         const bool events = !shp.copy_only && d.counts->events != 0;
         TileTotals t{};
-        if (events) t = tile_totals(d, shp, 0, 0, lds);
+        if (events) t = tile_totals<GROUPS>(d, shp, 0, 0, lds);
         if (threadIdx.x == 0) {
             DevCounts g = *d.counts;
             g.n_l_last = g.n_l;
@@ -2039,6 +2041,7 @@ __device__ __forceinline__ void finalize_scene(const DevState& d, const StepShap
 // the step of a scene each, the others write a compaction tile each. Neither
 // reads what the other writes (the counts are those of the other list
 // parity).
+template <bool GROUPS>
 __global__ __launch_bounds__(kScanThreads) void k_end_step(
     DevState d, StepShape sh, int nfin, const uint32_t* __restrict__ vals,
     const int* __restrict__ list_g, int* __restrict__ nlist_l, int* __restrict__ nlist_h,
@@ -2047,9 +2050,9 @@ __global__ __launch_bounds__(kScanThreads) void k_end_step(
     __shared__ int lds[kScanWaves][8];
     __shared__ int wsum[2][kScanItems][kScanWaves];
     if ((int)blockIdx.x < nfin)
-        finalize_scene(d, sh, (int)blockIdx.x, red, lds);
+        finalize_scene<GROUPS>(d, sh, (int)blockIdx.x, red, lds);
     else
-        compact_tile(d, sh, (int)blockIdx.x - nfin, vals, list_g, nlist_l, nlist_h, nlist_g, lds,
+        compact_tile<GROUPS>(d, sh, (int)blockIdx.x - nfin, vals, list_g, nlist_l, nlist_h, nlist_g, lds,
                      wsum);
 }
 
@@ -2704,9 +2707,10 @@ void launch_step(const DevState& base, const StepShape& sh, void* stream,
         k_tile_sums<<<sh.tile_groups, kScanThreads, 0, st>>>(d, sh);
     const int ntiles = sh.scan_tiles_l + sh.scan_tiles_h + sh.scan_tiles_g;
     auto end = [&](int nfin, int tiles) {
-        k_end_step<<<nfin + tiles, kScanThreads, 0, st>>>(d, sh, nfin, vals, d.list_g[par],
-                                                          d.list_l[par ^ 1], d.list_h[par ^ 1],
-                                                          d.list_g[par ^ 1]);
+        const auto k = sh.tile_groups ? k_end_step<true> : k_end_step<false>;
+        k<<<nfin + tiles, kScanThreads, 0, st>>>(d, sh, nfin, vals, d.list_g[par],
+                                                 d.list_l[par ^ 1], d.list_h[par ^ 1],
+                                                 d.list_g[par ^ 1]);
     };
     if (ev) {
         end(0, ntiles);
